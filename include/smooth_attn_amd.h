@@ -117,7 +117,7 @@ int sa_transpose16(const void* src, void* dst, int64_t rows, int64_t cols,
 
 /* Row kernel variants (sa_launch_info.variant). */
 enum {
-    SA_ROW_SCALAR = 0, /* element loads (unaligned rows or n_cols % vec != 0) */
+    SA_ROW_SCALAR = 0, /* element loads (unaligned rows or n_cols % vec != 0; norm: rows under 512 bytes of those) */
     SA_ROW_VEC = 1,    /* one wave per row, 16-byte loads */
     SA_ROW_SPLIT = 2   /* several waves per row, 16-byte loads */
 };

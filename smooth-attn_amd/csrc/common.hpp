@@ -150,6 +150,24 @@ __device__ __forceinline__ void store_words(T* p, const uint32_t* words) {
     store16(p, u32x4{words[0], words[1], words[2], words[3]});
 }
 
+
+// The same for rows that start at any multiple of the element size: one
+// 16-byte access at any 2-byte boundary (gfx950 global memory instructions
+// take any address; the wave still covers one contiguous span).
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+template <typename T>
+__device__ __forceinline__ void load_words_any(const T* p, uint32_t* words) {
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+    words[0] = v.x;
+    words[1] = v.y;
+    words[2] = v.z;
+    words[3] = v.w;
+}
+template <typename T>
+__device__ __forceinline__ void store_words_any(T* p, const uint32_t* words) {
+    __builtin_nontemporal_store(u32x4{words[0], words[1], words[2], words[3]}, reinterpret_cast<u32x4_any*>(p));
+}
+
 // Pack VEC = 16 / sizeof(T) floats into 4 words of T.
 template <typename T>
 __device__ __forceinline__ void pack_row16(const float* in, uint32_t* words) {

@@ -18,6 +18,8 @@
 //   dx = (alpha p / S') * (w / r) * (dy - T),  S' = sum w + 2^p eps,
 //   T = sum(dy w) / S'.
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace sa {
@@ -60,9 +62,37 @@ __device__ __forceinline__ void row_of_wave(int64_t w, int n_cols, bool causal, 
 }
 
 // ---------------------------------------------------------------------------
-// Vectorised kernels (rows 16-byte aligned, n_cols a multiple of VEC).
+// Vectorised kernels.  ANY = false: rows 16-byte aligned, n_cols a multiple of
+// VEC.  ANY = true: rows at any element address and any n_cols >= VEC.  There
+// each lane's 16 bytes are one access at element alignment, and the lane that
+// would run past the row's end is moved back to its last VEC columns: it then
+// recomputes some of its neighbour's columns (same bits, so either store may
+// win) and leaves them out of its share of the sums.
 // ---------------------------------------------------------------------------
-template <typename T, int NCH, int POWER>
+// First column of the lane whose place in the row is col0.
+template <bool ANY, int VEC>
+__device__ __forceinline__ int first_col(int col0, int n_cols) {
+    return ANY ? min(col0, n_cols - VEC) : col0;
+}
+// Whether the chunk at column c0 holds a column before `limit` (wave-uniform).
+// A moved-back lane may start before its chunk does.
+template <bool ANY, int VEC>
+__device__ __forceinline__ bool chunk_live(int c0, int limit, int n_cols) {
+    if constexpr (ANY) return c0 < n_cols && min(c0, n_cols - VEC) < limit;
+    return c0 < limit;
+}
+template <bool ANY, typename T>
+__device__ __forceinline__ void row_load(const T* p, uint32_t* words) {
+    if constexpr (ANY) load_words_any(p, words);
+    else load_words(p, words);
+}
+template <bool ANY, typename T>
+__device__ __forceinline__ void row_store(T* p, const uint32_t* words) {
+    if constexpr (ANY) store_words_any(p, words);
+    else store_words(p, words);
+}
+
+template <typename T, int NCH, int POWER, bool ANY = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fwd_waves<T, NCH>(), 8))) void norm_fwd_vec(const T* __restrict__ x, T* __restrict__ y,
                                                     int64_t n_rows, int n_cols, int64_t xs,
                                                     int64_t ys, int causal, float alpha,
@@ -87,8 +117,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
-        if (c * 64 * VEC < limit) {
-            load_words(xr + (col0 < limit ? col0 : 0), raw[c]);
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
+            row_load<ANY>(xr + (cb < limit ? cb : 0), raw[c]);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) raw[c][k] = 0u;
@@ -100,16 +131,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) w[c][e] = 0.f;
-        if (c * 64 * VEC < limit) {
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const float a = __builtin_fmaf(alpha, elem<T>(raw[c], e), neg_alpha_theta);
                 const float t = a + fast_sqrt(__builtin_fmaf(a, a, 4.f));
-                const float wv = (col0 + e <= qpos) ? power_of<POWER>(t) : 0.f;
+                const float wv = (cb + e <= qpos) ? power_of<POWER>(t) : 0.f;
                 w[c][e] = wv;
-                part += wv;
+                part += !ANY || cb + e >= col0 ? wv : 0.f;
             }
         }
     }
@@ -118,18 +150,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
         if (col0 < n_cols) {
             float ov[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ov[e] = w[c][e] * inv;
             uint32_t packed[4];
             pack_row16<T>(ov, packed);
-            store_words(yr + col0, packed);
+            row_store<ANY>(yr + cb, packed);
         }
     }
 }
 
-template <typename T, typename TG, int NCH, int POWER>
+template <typename T, typename TG, int NCH, int POWER, bool ANY = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T, TG, NCH>(), 8))) void norm_bwd_vec(const T* __restrict__ x, const TG* __restrict__ dy,
                                                     T* __restrict__ dx, int64_t n_rows, int n_cols,
                                                     int64_t xs, int64_t gs, int64_t dxs, int causal,
@@ -153,11 +186,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
-        if (c * 64 * VEC < limit) {
-            const int off = col0 < limit ? col0 : 0;
-            load_words(xr + off, rx[c]);
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
+            const int off = cb < limit ? cb : 0;
+            row_load<ANY>(xr + off, rx[c]);
 #pragma unroll
-            for (int k = 0; k < GW; ++k) load_words(gr + off + k * (16 / sizeof(TG)), &rg[c][4 * k]);
+            for (int k = 0; k < GW; ++k) row_load<ANY>(gr + off + k * (16 / sizeof(TG)), &rg[c][4 * k]);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) rx[c][k] = 0u;
@@ -173,20 +207,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) q[c][e] = 0.f;
-        if (c * 64 * VEC < limit) {
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
-                const bool live = col0 + e <= qpos;
+                const bool live = cb + e <= qpos;
+                const bool own = !ANY || cb + e >= col0;  // counted by this lane
                 const float a = __builtin_fmaf(alpha, elem<T>(rx[c], e), neg_alpha_theta);
                 const float s = __builtin_fmaf(a, a, 4.f);
                 const float rr = fast_rsqrt(s);
                 const float t = __builtin_fmaf(s, rr, a);  // a + sqrt(s)
                 const float wv = live ? power_of<POWER>(t) : 0.f;
                 q[c][e] = wv * rr;
-                s_part += wv;
-                u_part = live ? __builtin_fmaf(elem<TG>(rg[c], e), wv, u_part) : u_part;
+                s_part += own ? wv : 0.f;
+                u_part = live && own ? __builtin_fmaf(elem<TG>(rg[c], e), wv, u_part) : u_part;
             }
         }
     }
@@ -198,16 +234,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
         if (col0 < n_cols) {
             float ov[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const float d = (C * q[c][e]) * (elem<TG>(rg[c], e) - Tdot);
-                ov[e] = (col0 + e <= qpos) ? d : 0.f;
+                ov[e] = (cb + e <= qpos) ? d : 0.f;
             }
             uint32_t packed[4];
             pack_row16<T>(ov, packed);
-            store_words(dxr + col0, packed);
+            row_store<ANY>(dxr + cb, packed);
         }
     }
 }
@@ -221,7 +258,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T
 template <int R>
 constexpr int split_block_waves() { return R > kWavesPerBlock ? R : kWavesPerBlock; }
 
-template <typename T, int NCH, int POWER, int R>
+template <typename T, int NCH, int POWER, int R, bool ANY = false>
 __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_fwd_split(const T* __restrict__ x, T* __restrict__ y, int64_t n_rows,
                                                       int n_cols, int64_t xs, int64_t ys, int causal, float alpha,
                                                       float neg_alpha_theta, float eps_scaled) {
@@ -244,8 +281,9 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_fwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
-        if (c * 64 * VEC < limit) {
-            load_words(xr + (col0 < limit ? col0 : 0), raw[i]);
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
+            row_load<ANY>(xr + (cb < limit ? cb : 0), raw[i]);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) raw[i][k] = 0u;
@@ -257,16 +295,17 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_fwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) w[i][e] = 0.f;
-        if (c * 64 * VEC < limit) {
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const float a = __builtin_fmaf(alpha, elem<T>(raw[i], e), neg_alpha_theta);
                 const float t = a + fast_sqrt(__builtin_fmaf(a, a, 4.f));
-                const float wv = (col0 + e <= qpos) ? power_of<POWER>(t) : 0.f;
+                const float wv = (cb + e <= qpos) ? power_of<POWER>(t) : 0.f;
                 w[i][e] = wv;
-                part += wv;
+                part += !ANY || cb + e >= col0 ? wv : 0.f;
             }
         }
     }
@@ -282,18 +321,19 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_fwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
         if (col0 < n_cols) {
             float ov[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ov[e] = w[i][e] * inv;
             uint32_t packed[4];
             pack_row16<T>(ov, packed);
-            store_words(yr + col0, packed);
+            row_store<ANY>(yr + cb, packed);
         }
     }
 }
 
-template <typename T, typename TG, int NCH, int POWER, int R>
+template <typename T, typename TG, int NCH, int POWER, int R, bool ANY = false>
 __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_bwd_split(const T* __restrict__ x, const TG* __restrict__ dy,
                                                       T* __restrict__ dx, int64_t n_rows, int n_cols, int64_t xs,
                                                       int64_t gs, int64_t dxs, int causal, float alpha,
@@ -320,11 +360,12 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_bwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
-        if (c * 64 * VEC < limit) {
-            const int off = col0 < limit ? col0 : 0;
-            load_words(xr + off, rx[i]);
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
+            const int off = cb < limit ? cb : 0;
+            row_load<ANY>(xr + off, rx[i]);
 #pragma unroll
-            for (int k = 0; k < GW; ++k) load_words(gr + off + k * (16 / sizeof(TG)), &rg[i][4 * k]);
+            for (int k = 0; k < GW; ++k) row_load<ANY>(gr + off + k * (16 / sizeof(TG)), &rg[i][4 * k]);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) rx[i][k] = 0u;
@@ -338,20 +379,22 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_bwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) q[i][e] = 0.f;
-        if (c * 64 * VEC < limit) {
+        if (chunk_live<ANY, VEC>(c * 64 * VEC, limit, n_cols)) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
-                const bool live = col0 + e <= qpos;
+                const bool live = cb + e <= qpos;
+                const bool own = !ANY || cb + e >= col0;  // counted by this lane
                 const float a = __builtin_fmaf(alpha, elem<T>(rx[i], e), neg_alpha_theta);
                 const float s = __builtin_fmaf(a, a, 4.f);
                 const float rr = fast_rsqrt(s);
                 const float t = __builtin_fmaf(s, rr, a);
                 const float wv = live ? power_of<POWER>(t) : 0.f;
                 q[i][e] = wv * rr;
-                s_part += wv;
-                u_part = live ? __builtin_fmaf(elem<TG>(rg[i], e), wv, u_part) : u_part;
+                s_part += own ? wv : 0.f;
+                u_part = live && own ? __builtin_fmaf(elem<TG>(rg[i], e), wv, u_part) : u_part;
             }
         }
     }
@@ -375,23 +418,24 @@ __global__ __launch_bounds__(64 * split_block_waves<R>()) void norm_bwd_split(co
     for (int i = 0; i < NW; ++i) {
         const int c = wr + R * i;
         const int col0 = (c * 64 + lane) * VEC;
+        const int cb = first_col<ANY, VEC>(col0, n_cols);
         if (col0 < n_cols) {
             float ov[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const float d = (C * q[i][e]) * (elem<TG>(rg[i], e) - Tdot);
-                ov[e] = (col0 + e <= qpos) ? d : 0.f;
+                ov[e] = (cb + e <= qpos) ? d : 0.f;
             }
             uint32_t packed[4];
             pack_row16<T>(ov, packed);
-            store_words(dxr + col0, packed);
+            row_store<ANY>(dxr + cb, packed);
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// Scalar kernels for rows that are not 16-byte aligned: one wave per row,
-// element-strided passes over global memory (no register cache).
+// Element kernels for short rows that are not 16-byte aligned: one wave per
+// row, element-strided passes over global memory (no register cache).
 // ---------------------------------------------------------------------------
 template <typename T, int POWER>
 __global__ __launch_bounds__(256) void norm_fwd_scalar(const T* __restrict__ x, T* __restrict__ y,
@@ -487,11 +531,29 @@ int chunks_for(int n_cols, int vec) {
     return nch;
 }
 
+// Whether rows that are not 16-byte aligned (or whose length is no multiple
+// of VEC) take the ANY kernels: from 512 bytes per row, where a split-row grid
+// still fits (the element kernels take more rows).  Element loads moved 2 or
+// 4 bytes per lane and read x twice; causal [2,16,L,L] bf16, forward /
+// backward, element -> ANY: L = 1023 55.0 / 58.4 -> 20.3 / 27.7 us (L = 1024,
+// aligned, 18.4 / 24.7 us), L = 257 (n = 256 matrices) 25.5 / 32.2 -> 21.7 /
+// 29.4 us; one [4095,4095] 43.2 / 47.8 -> 13.2 / 16.4 us; row-wise fp32 at
+// 1023 columns 91.6 -> 47.9 us, at 129 12.9 -> 9.9 us.  Below, a row fills a
+// fraction of one wave's lanes and the element kernels win: bf16 at 129
+// columns 10.4 / 12.1 vs 11.7 / 16.3 us.
+constexpr int kAnyRowBytes = 512;
+bool any_rows_ok(int64_t n_rows, int n_cols, int nch, int elem_bytes) {
+    const int R = split_for(nch);
+    const dim3 sg = R == 8 ? split_grid<8>(n_rows) : R == 4 ? split_grid<4>(n_rows) : split_grid<1>(n_rows);
+    return n_cols * elem_bytes >= kAnyRowBytes && grid_fits(sg, dim3(64 * std::max(R, kWavesPerBlock)));
+}
+
 float eps_for_power(int power) { return kEps * static_cast<float>(1 << power); }
 
-// The forward launch for these arguments: element kernel for unaligned rows
-// (or n_cols not a multiple of the vector width), else one wave per row, or
-// split_for(NCH) waves per row for long rows.
+// The forward launch for these arguments: one wave per row, or split_for(NCH)
+// waves per row for long rows, with any-address accesses for unaligned rows
+// (or n_cols not a multiple of the vector width); element kernel for short
+// ones of those.
 template <typename T, int POWER>
 int plan_fwd_t(const void* x, const void* y, int64_t n_rows, int n_cols, int64_t xs, int64_t ys, RowLaunch& L) {
     constexpr int VEC = 16 / sizeof(T);
@@ -500,14 +562,14 @@ int plan_fwd_t(const void* x, const void* y, int64_t n_rows, int n_cols, int64_t
     L.rows_per_block = kWavesPerBlock;
     L.waves_per_row = 1;
     const bool vec_ok = (n_cols % VEC == 0) && (xs % VEC == 0) && (ys % VEC == 0) && aligned16(x) && aligned16(y);
-    if (!vec_ok) {
+    const int nch = chunks_for(n_cols, VEC);
+    if (!vec_ok && !any_rows_ok(n_rows, n_cols, nch, sizeof(T))) {
         L.fn = reinterpret_cast<const void*>(&norm_fwd_scalar<T, POWER>);
         L.variant = SA_ROW_SCALAR;
         L.elems_per_load = 1;
         L.row_pass_elems = 64;
         return 0;
     }
-    const int nch = chunks_for(n_cols, VEC);
     L.elems_per_load = VEC;
     L.row_pass_elems = nch * 64 * VEC;
     switch (nch) {
@@ -515,14 +577,16 @@ int plan_fwd_t(const void* x, const void* y, int64_t n_rows, int n_cols, int64_t
     case N:                                                                                   \
         if constexpr (split_for(N) > 1) {                                                     \
             constexpr int R = split_for(N);                                                   \
-            L.fn = reinterpret_cast<const void*>(&norm_fwd_split<T, N, POWER, R>);            \
+            L.fn = vec_ok ? reinterpret_cast<const void*>(&norm_fwd_split<T, N, POWER, R>)    \
+                          : reinterpret_cast<const void*>(&norm_fwd_split<T, N, POWER, R, true>); \
             L.grid = split_grid<R>(n_rows);                                                   \
             L.block = dim3(64 * split_block_waves<R>());                                      \
             L.rows_per_block = split_block_waves<R>() / R;                                    \
             L.waves_per_row = R;                                                              \
             L.variant = SA_ROW_SPLIT;                                                         \
         } else {                                                                              \
-            L.fn = reinterpret_cast<const void*>(&norm_fwd_vec<T, N, POWER>);                 \
+            L.fn = vec_ok ? reinterpret_cast<const void*>(&norm_fwd_vec<T, N, POWER>)         \
+                          : reinterpret_cast<const void*>(&norm_fwd_vec<T, N, POWER, true>);  \
             L.variant = SA_ROW_VEC;                                                           \
         }                                                                                     \
         return 0;
@@ -578,24 +642,33 @@ int launch_bwd_t(const void* x, const void* dy, void* dx, int64_t n_rows, int n_
     T* dp = static_cast<T*>(dx);
     const bool vec_ok = (n_cols % VEC == 0) && (xs % VEC == 0) && (gs % GVEC == 0) && (dxs % VEC == 0) &&
                         aligned16(x) && aligned16(dy) && aligned16(dx);
-    if (!vec_ok) {
+    const int nch = chunks_for(n_cols, VEC);
+    if (!vec_ok && !any_rows_ok(n_rows, n_cols, nch, sizeof(T))) {
         if (!grid_fits(grid, block)) return SA_ERR_BAD_SHAPE;
         norm_bwd_scalar<T, TG, POWER><<<grid, block, 0, st>>>(xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal,
                                                               alpha, nat, eps);
         return status_from_launch();
     }
-    switch (chunks_for(n_cols, VEC)) {
+    switch (nch) {
 #define SA_BWD_CASE(N)                                                                                   \
     case N:                                                                                              \
         if constexpr (split_for(N) > 1) {                                                                \
             const dim3 sg = split_grid<split_for(N)>(n_rows), sb(64 * split_block_waves<split_for(N)>()); \
             if (!grid_fits(sg, sb)) return SA_ERR_BAD_SHAPE;                                             \
-            norm_bwd_split<T, TG, N, POWER, split_for(N)><<<sg, sb, 0, st>>>(                            \
-                    xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal, alpha, nat, eps);                   \
+            if (vec_ok)                                                                                  \
+                norm_bwd_split<T, TG, N, POWER, split_for(N)><<<sg, sb, 0, st>>>(                        \
+                        xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal, alpha, nat, eps);               \
+            else                                                                                         \
+                norm_bwd_split<T, TG, N, POWER, split_for(N), true><<<sg, sb, 0, st>>>(                  \
+                        xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal, alpha, nat, eps);               \
         } else {                                                                                         \
             if (!grid_fits(grid, block)) return SA_ERR_BAD_SHAPE;                                        \
-            norm_bwd_vec<T, TG, N, POWER><<<grid, block, 0, st>>>(xp, gp, dp, n_rows, n_cols, xs, gs, dxs, \
-                                                                  causal, alpha, nat, eps);              \
+            if (vec_ok)                                                                                  \
+                norm_bwd_vec<T, TG, N, POWER><<<grid, block, 0, st>>>(                                   \
+                        xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal, alpha, nat, eps);               \
+            else                                                                                         \
+                norm_bwd_vec<T, TG, N, POWER, true><<<grid, block, 0, st>>>(                             \
+                        xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal, alpha, nat, eps);               \
         }                                                                                                \
         break;
         SA_BWD_CASE(1)
