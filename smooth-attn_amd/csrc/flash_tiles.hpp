@@ -21,8 +21,8 @@ __device__ __forceinline__ void tile_dma16(__amdgpu_buffer_rsrc_t rs, int voff, 
 }
 
 // Per-lane byte offset past the buffer resource of every tile the attention
-// kernels load (their tiles span at most 64 rows of under 2^25 bytes, so a
-// resource holds at most 2^31 - 1024 bytes): the lane's load returns zeros.
+// kernels load (their tiles span at most 64 rows of under 2^25 bytes, or 128
+// of at most 2^23, so a resource holds at most 2^31 - 1024 bytes): the lane's load returns zeros.
 // Lanes whose 16-byte chunk lies past the tensors' head dim take it.
 constexpr int kPastTile = 0x7FFFFFF0;
 
