@@ -6,10 +6,10 @@
 //   (reference kernels.py:2681-2773 and the decode references of
 //    tests/test_paged_long_context.py:39-65)
 //
-// Work split (stream-K style, balanced whatever the context lengths): a
-// plan kernel counts each sequence's 32-token tiles, prefix-sums them over
-// (sequence, KV head) in that order and fixes the number of active waves
-// Ne; a persistent grid of one-wave blocks then gives wave w the tiles
+// Work split (stream-K style, balanced whatever the context lengths): a plan
+// counts each sequence's 32-token tiles, prefix-sums them over (sequence, KV
+// head) in that order and fixes the number of active waves Ne (every wave
+// works it out, or for large batches a kernel: WavePlan); a persistent grid of one-wave blocks then gives wave w the tiles
 // [floor(w Tt / Ne), floor((w+1) Tt / Ne)) of the Tt in total.  A wave's
 // range is cut at (sequence, KV head) boundaries into pieces; each piece is
 // walked in tiles of 32 tokens, reading every K/V row once for all G query
@@ -62,6 +62,77 @@ __device__ __forceinline__ int ctx_of(const PagedParams& p, int b) {
     return min(max(p.ctx[b], 0), p.max_pages * p.P);
 }
 
+// Tiles of sequence b's segments (all KV heads) for context length ctx.
+__device__ __forceinline__ int tiles_of(const PagedParams& p, int ctx) {
+    return p.Hkv * ((ctx + kTile - 1) / kTile);
+}
+
+// Waves that get work (see paged_plan_kernel).
+__device__ __forceinline__ int active_waves(const PagedParams& p, int tiles) {
+    return tiles == 0 ? 0 : max(1, min(p.n_waves, tiles / p.per));
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave.
+__device__ __forceinline__ int wave_prefix(int v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(v, off);
+        v += lane >= off ? u : 0;
+    }
+    return v;
+}
+
+// The plan as one wave sees it.  Up to kRegSeqs sequences every wave works
+// the plan out for itself, lane b holding sequence b: one load of the context
+// lengths and a wave scan, where the plan kernel costs a launch and the
+// waves a chain of dependent loads of what it wrote.  With the merge below, 8
+// sequences of 64 to 2048 tokens (Hq 32 / Hkv 8, D 128) 26.8 -> 17.8 us, one
+// of 16384 24.1 -> 13.9 us, 64 of 512 to 16384 tokens 1% faster; the same
+// bits.  Larger batches (one lane would hold several sequences) read the plan
+// kernel's, 2% of the time at 100 sequences.
+constexpr int kRegSeqs = 64;
+struct WavePlan {
+    const PagedParams& p;
+    bool regs;      // wave-uniform
+    int ctx, last;  // lane b: context length of sequence b, plan[b + 1]
+    int Tt, Ne;
+    __device__ __forceinline__ explicit WavePlan(const PagedParams& prm) : p(prm), regs(prm.B <= kRegSeqs) {
+        if (regs) {
+            const int b = threadIdx.x & 63;
+            ctx = b < p.B ? ctx_of(p, b) : 0;
+            last = wave_prefix(tiles_of(p, ctx));
+            Tt = __builtin_amdgcn_readlane(last, 63);
+            Ne = active_waves(p, Tt);
+        } else {
+            ctx = last = 0;
+            Tt = p.plan[p.B];
+            Ne = p.plan[p.B + 1];
+        }
+    }
+    // plan[b + 1], plan[b] and the context length of sequence b (wave-uniform)
+    __device__ __forceinline__ int end(int b) const { return regs ? __builtin_amdgcn_readlane(last, b) : p.plan[b + 1]; }
+    __device__ __forceinline__ int begin(int b) const {
+        return regs ? (b == 0 ? 0 : __builtin_amdgcn_readlane(last, b - 1)) : p.plan[b];
+    }
+    __device__ __forceinline__ int context(int b) const {
+        return regs ? __builtin_amdgcn_readlane(ctx, b) : ctx_of(p, b);
+    }
+    // The sequence that tile x < Tt belongs to.
+    __device__ __forceinline__ int sequence_of(int x) const {
+        const int lane = threadIdx.x & 63;
+        if (regs) return __builtin_ctzll(__ballot(lane < p.B && last > x));
+        int b = 0;
+        for (int b0 = 0; b0 < p.B; b0 += 64) {
+            const int bi = b0 + lane;
+            const unsigned long long m = __ballot(bi < p.B && p.plan[bi] <= x);
+            if (m == 0) break;
+            b = b0 + 63 - __builtin_clzll(m);
+        }
+        return b;
+    }
+};
+
 // Plan: plan[b] = sum_{b' < b} Hkv * ceil(ctx_b' / 32) for b <= B (plan[B] =
 // Tt, the tiles of all (sequence, KV head) segments), plan[B + 1] = Ne, the
 // waves that get work: every wave's range holds at least `per` tiles (so a
@@ -73,7 +144,7 @@ __global__ __launch_bounds__(256) void paged_plan_kernel(PagedParams p) {
     int carry = 0;
     for (int b0 = 0; b0 < p.B; b0 += 256) {
         const int b = b0 + tid;
-        const int n = b < p.B ? p.Hkv * ((ctx_of(p, b) + kTile - 1) / kTile) : 0;
+        const int n = b < p.B ? tiles_of(p, ctx_of(p, b)) : 0;
         part[tid] = n;
         __syncthreads();
         // inclusive scan of part[] (Hillis-Steele)
@@ -89,7 +160,7 @@ __global__ __launch_bounds__(256) void paged_plan_kernel(PagedParams p) {
     }
     if (tid == 0) {
         p.plan[p.B] = carry;
-        p.plan[p.B + 1] = carry == 0 ? 0 : max(1, min(p.n_waves, carry / p.per));
+        p.plan[p.B + 1] = active_waves(p, carry);
     }
 }
 
@@ -201,34 +272,25 @@ __global__ __launch_bounds__(64 * WPB) void paged_partial_kernel(PagedParams p) 
     const int hi = lane >> 5;
     const int l32 = lane & 31;
     const int w = blockIdx.x;
-    const int Tt = p.plan[p.B];
-    const int Ne = p.plan[p.B + 1];
+    const WavePlan plan(p);
+    const int Tt = plan.Tt, Ne = plan.Ne;
     if (w >= Ne) return;  // no work for this wave (tiny problems)
     const int x_end = static_cast<int>(static_cast<int64_t>(w + 1) * Tt / Ne);
     int x = static_cast<int>(static_cast<int64_t>(w) * Tt / Ne);
     const int logP = p.logP;
     const int pmask = p.P - 1;
 
-    // Sequence b of tile x: the last b with plan[b] <= x (plan[b] ascending).
-    int b = 0;
-    for (int b0 = 0; b0 < p.B; b0 += 64) {
-        const int bi = b0 + lane;
-        const bool le = bi < p.B && p.plan[bi] <= x;
-        const unsigned long long m = __ballot(le);
-        if (m == 0) break;
-        b = b0 + 63 - __builtin_clzll(m);
-    }
-
+    int b = plan.sequence_of(x);
     while (x < x_end) {
         // Segment (b, hk) holding tile x; skip sequences with no tiles.
-        while (p.plan[b + 1] <= x) ++b;
-        const int seg0 = p.plan[b];
-        const int n_b = (p.plan[b + 1] - seg0) / p.Hkv;  // tiles per KV head of b
+        while (plan.end(b) <= x) ++b;
+        const int seg0 = plan.begin(b);
+        const int n_b = (plan.end(b) - seg0) / p.Hkv;  // tiles per KV head of b
         const int rel = x - seg0;
         const int hk = rel / n_b;
         const int seg_start = seg0 + hk * n_b;
         const int piece_end = min(x_end, seg_start + n_b);
-        const int ctx = ctx_of(p, b);
+        const int ctx = plan.context(b);
         const int t_begin = (x - seg_start) * kTile;
         const int t_end = min(ctx, (piece_end - seg_start) * kTile);
         // slot: this wave minus the owner of the segment's first tile
@@ -457,30 +519,47 @@ __global__ __launch_bounds__(64 * WPB) void paged_partial_kernel(PagedParams p) 
 }
 
 // Sum the piece partials of one (b, query head) in slot order, then divide
-// (an empty context gives 0 / eps = 0).
+// (an empty context gives 0 / eps = 0).  Bound by memory latency: up to
+// kMergeRun slots are read before the first is added (one at a time, 8
+// sequences of 64 to 2048 tokens took 9.6 us here).
+constexpr int kMergeRun = 16;
 template <int D>
-__global__ __launch_bounds__(D) void paged_merge_kernel(PagedParams p) {
+__global__ __launch_bounds__(D < 64 ? 64 : D) void paged_merge_kernel(PagedParams p) {
     const int bh = blockIdx.x;
     const int b = bh / p.Hq;
     const int hq = bh - b * p.Hq;
     const int hk = hq / p.G;
     const int d = threadIdx.x;
-    const int Tt = p.plan[p.B];
-    const int Ne = p.plan[p.B + 1];
-    const int seg0 = p.plan[b];
-    const int n_b = (p.plan[b + 1] - seg0) / p.Hkv;
+    const WavePlan plan(p);
+    const int seg0 = plan.begin(b);
+    const int n_b = (plan.end(b) - seg0) / p.Hkv;
     float o = 0.f, s = 0.f;
     if (n_b > 0) {
         const int first = seg0 + hk * n_b, last = first + n_b - 1;
-        const int w0 = static_cast<int>((static_cast<int64_t>(first + 1) * Ne - 1) / Tt);
-        const int w1 = static_cast<int>((static_cast<int64_t>(last + 1) * Ne - 1) / Tt);
+        const int w0 = static_cast<int>((static_cast<int64_t>(first + 1) * plan.Ne - 1) / plan.Tt);
+        const int w1 = static_cast<int>((static_cast<int64_t>(last + 1) * plan.Ne - 1) / plan.Tt);
+        const int n = w1 - w0 + 1;
         const int64_t slot0 = static_cast<int64_t>(bh) * p.n_slots;
-        for (int i = 0; i <= w1 - w0; ++i) {
-            o += p.ws_o[(slot0 + i) * p.D + d];
-            s += p.ws_s[slot0 + i];
+        const float* wo = p.ws_o + slot0 * p.D + min(d, p.D - 1);
+        const float* ws = p.ws_s + slot0;
+        for (int i0 = 0; i0 < n; i0 += 64) {
+            const int m = min(n - i0, 64);
+            const float sl = ws[i0 + min(d & 63, m - 1)];  // lane l: the sum of slot i0 + l
+            for (int i = 0; i < m; i += kMergeRun) {
+                float po[kMergeRun];
+#pragma unroll
+                for (int j = 0; j < kMergeRun; ++j) po[j] = wo[static_cast<int64_t>(i0 + min(i + j, m - 1)) * p.D];
+#pragma unroll
+                for (int j = 0; j < kMergeRun; ++j) {
+                    if (i + j < m) {
+                        o += po[j];
+                        s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sl), i + j));
+                    }
+                }
+            }
         }
     }
-    p.out[b * p.os[0] + hq * p.os[1] + d * p.os[2]] = static_cast<bf16>(o / (s + kEps));
+    if (d < p.D) p.out[b * p.os[0] + hq * p.os[1] + d * p.os[2]] = static_cast<bf16>(o / (s + kEps));
 }
 
 // Blocks of paged_partial_kernel<QE, CE, D, U, WPB> resident on the device at
@@ -521,12 +600,12 @@ int launch_paged(PagedParams prm, hipStream_t st) {
     const int64_t max_tiles = static_cast<int64_t>(prm.B) * prm.Hkv *
                               ((static_cast<int64_t>(prm.max_pages) * prm.P + kTile - 1) / kTile);
     prm.n_waves = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(resident, max_tiles / prm.per)));
-    paged_plan_kernel<<<1, 256, 0, st>>>(prm);
+    if (prm.B > kRegSeqs) paged_plan_kernel<<<1, 256, 0, st>>>(prm);
     if (uniform)
         paged_partial_kernel<QE, CE, D, true, WPB><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
     else
         paged_partial_kernel<QE, CE, D, false, WPB><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
-    paged_merge_kernel<D><<<static_cast<unsigned>(prm.B) * prm.Hq, prm.D, 0, st>>>(prm);
+    paged_merge_kernel<D><<<static_cast<unsigned>(prm.B) * prm.Hq, (prm.D + 63) / 64 * 64, 0, st>>>(prm);
     return status_from_launch();
 }
 
