@@ -88,6 +88,9 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+_host = None
+_HOST_PATH = Path(__file__).resolve().parent / "_host.so"
+_BUILD = "build it with `python -c 'import __graft_entry__ as g; g.build()'` from the repository root"
 
 
 def load():
@@ -100,8 +103,7 @@ def load():
             return _lib
         if not LIB_PATH.exists():
             raise RuntimeError(
-                f"smooth_attn HIP library not found at {LIB_PATH}; build it with "
-                "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root"
+                f"smooth_attn HIP library not found at {LIB_PATH}; {_BUILD}"
             )
         lib = ctypes.CDLL(str(LIB_PATH))
         for name, (res, args) in SIGNATURES.items():
@@ -110,6 +112,28 @@ def load():
             fn.argtypes = args
         _lib = lib
         return lib
+
+
+def host():
+    """The native call path (csrc/host/host.cpp), loaded once and bound to the
+    library's functions."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is not None:
+            return _host
+        if not _HOST_PATH.exists():
+            raise RuntimeError(f"smooth_attn host extension not found at {_HOST_PATH}; {_BUILD}")
+        import importlib.util
+
+        spec = importlib.util.spec_from_file_location(f"{__package__}._host", _HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
+        _host = mod
+        return mod
 
 
 def check(status: int, what: str) -> None:

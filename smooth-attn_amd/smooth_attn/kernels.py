@@ -99,10 +99,20 @@ BENCH_POWER = DEFAULT_FAMILY.power
 # ---------------------------------------------------------------------------
 def _resolve_family(alpha, theta, power, family):
     if family is None:
+        if alpha is DEFAULT_FAMILY.alpha and theta is DEFAULT_FAMILY.theta and power is DEFAULT_FAMILY.power:
+            return DEFAULT_FAMILY
         return FamilyConfig(alpha=alpha, theta=theta, power=power)
     if (alpha, theta, power) != (DEFAULT_FAMILY.alpha, DEFAULT_FAMILY.theta, DEFAULT_FAMILY.power):
         raise ValueError("pass either family=... or alpha/theta/power overrides, not both")
     return family
+
+
+def _native():
+    """The native call path (csrc/host/host.cpp).  It takes the calls whose
+    tensors the kernels can use as they are and answers None (or False) to
+    every other one, which then goes through the Python path below it; on a
+    machine without a GPU nothing is ordinary, and the Python path raises."""
+    return _lib.host()
 
 
 def _validate_cuda_tensor(x, *, name):
@@ -278,7 +288,8 @@ def softplus_norm_triton(x, alpha=DEFAULT_FAMILY.alpha, theta=DEFAULT_FAMILY.the
     family = _resolve_family(alpha, theta, power, family)
     x_row = _prepare_rowwise_input(x)
     out = torch.empty_like(x_row)
-    _norm_fwd_2d(x_row, out, family, causal=False)
+    if not _native().norm_out(out, x_row, False, family.alpha, family.theta, family.power):
+        _norm_fwd_2d(x_row, out, family, causal=False)
     if return_meta:
         return out, _row_launch_meta("softplus_norm", "norm", x_row, out,
                                      lambda: _norm_fwd_2d(x_row, out, family, causal=False), family.power)
@@ -289,6 +300,8 @@ def softplus_norm_triton_out(out, x, alpha=DEFAULT_FAMILY.alpha, theta=DEFAULT_F
                              power=DEFAULT_FAMILY.power, *, family=None, return_meta=False):
     """Row-wise forward into ``out`` — kernels.py:1006-1031."""
     family = _resolve_family(alpha, theta, power, family)
+    if not return_meta and _native().norm_out(out, x, False, family.alpha, family.theta, family.power):
+        return out
     x_row = _prepare_rowwise_input(x)
     kernel_out, user_out = _prepare_output(out, x_row)
     _norm_fwd_2d(x_row, kernel_out, family, causal=False)
@@ -314,6 +327,8 @@ def softplus_norm_causal_triton_out(out, x, alpha=DEFAULT_FAMILY.alpha, theta=DE
     chunk skipping and in-kernel zero fill.
     """
     family = _resolve_family(alpha, theta, power, family)
+    if not return_meta and _native().norm_out(out, x, True, family.alpha, family.theta, family.power):
+        return out
     x_attn = _prepare_attention_input(x)
     kernel_out, user_out = _prepare_output(out, x_attn)
     seq_len = x_attn.shape[-1]
@@ -395,6 +410,9 @@ def softplus_norm_causal(x, alpha=DEFAULT_FAMILY.alpha, theta=DEFAULT_FAMILY.the
     eager formula in fp32, cast back to x's dtype."""
     family = _resolve_family(alpha, theta, power, family)
     if implementation == "triton":
+        y = _native().causal_norm(x, family.alpha, family.theta, family.power)
+        if y is not None:
+            return y
         return _SoftplusNormCausalAutogradFn.apply(x, family.alpha, family.theta, family.power)
     if implementation == "eager":
         return softplus_norm_causal_eager(x.float(), family=family).to(x.dtype)
@@ -684,6 +702,9 @@ class _SP2NormFlashAttentionFn(torch.autograd.Function):
 def sp2norm_flash_attention(q, k, v, *, scale=None, window_size=0, exact_math=False):
     """Fused causal squareplus attention with autograd, GQA and sliding
     windows — kernels.py:2016-2050."""
+    o = _native().flash(q, k, v, scale, window_size, exact_math)
+    if o is not None:
+        return o
     assert q.ndim == 4 and k.ndim == 4 and v.ndim == 4
     B, H_q, T, D = q.shape
     H_kv = k.shape[1]
@@ -1003,6 +1024,9 @@ def _paged_dtype_code(q_dtype, k_dtype, v_dtype):
 
 def sp2norm_paged_attention(q, k_cache, v_cache, block_table, context_lens, *, scale=None, block_size=16):
     """Paged single-token decode — kernels.py:2776-2829 (output bf16 [B, Hq, D])."""
+    out = _native().paged(q, k_cache, v_cache, block_table, context_lens, scale, block_size)
+    if out is not None:
+        return out
     assert q.ndim == 4 and q.shape[2] == 1, "Decode: q must be [B, H, 1, D]"
     B, H_q, _, D = q.shape
     H_kv = k_cache.shape[1]
@@ -1061,6 +1085,9 @@ def sp2norm_paged_kv_append(k_cache, v_cache, k_new, v_new, block_table, context
     k_new, v_new: [B, Hkv, n_new, D]; caches [n_pages, Hkv, block_size, D].
     No counterpart in the reference, which builds its caches with Python
     loops (tests/test_paged_attention.py:10-73)."""
+    new_lens = _native().paged_append(k_cache, v_cache, k_new, v_new, block_table, context_lens, block_size)
+    if new_lens is not None:
+        return new_lens
     assert k_new.ndim == 4 and v_new.shape == k_new.shape
     B, H_kv, n_new, D = k_new.shape
     assert k_cache.shape[1] == H_kv and k_cache.shape[3] == D and v_cache.shape == k_cache.shape

@@ -1,0 +1,315 @@
+"""The native call path against the Python path: same bits, same gradients, same
+refusals, over the forms of calls that either may get; and what sits between a
+call and the device (no_grad, saved-tensor hooks, checkpointing, functorch,
+forward mode, tensor subclasses, modes, threads, streams)."""
+import threading
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwad
+from torch.utils.checkpoint import checkpoint
+
+import smooth_attn
+from smooth_attn import _lib, kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+class _NoNative:
+    """Answers as the native path does to a call it does not take."""
+
+    def __init__(self):
+        self.asked = 0
+
+    def _none(self, *a):
+        self.asked += 1
+
+    causal_norm = flash = paged = paged_append = _none
+
+    def norm_out(self, *a):
+        self.asked += 1
+        return False
+
+
+class _Counting:
+    """The native path, counting the calls that it took."""
+
+    def __init__(self):
+        self.took = 0
+
+    def __getattr__(self, name):
+        fn = getattr(_lib.host(), name)
+
+        def call(*a):
+            r = fn(*a)
+            self.took += r is not None and name != "norm_out"  # (the Python path asks for that one too)
+            return r
+        return call
+
+
+def both(monkeypatch, call):
+    """call() on the Python path and on the native one: (Python, native, times the native path took it)."""
+    got = []
+    for nat in (_NoNative(), _Counting()):
+        monkeypatch.setattr(kernels, "_native", lambda nat=nat: nat)
+        try:
+            got.append(call())
+        except Exception as e:  # noqa: BLE001
+            got.append(e)
+    monkeypatch.undo()
+    return got[0], got[1], nat.took
+
+
+def same(a, b):
+    if isinstance(a, Exception) or isinstance(b, Exception):
+        assert type(a) is type(b), (a, b)
+        return
+    if isinstance(a, torch.Tensor):
+        assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+        assert a.requires_grad == b.requires_grad and type(a) is type(b)
+        a, b = (torch.empty(t.numel(), dtype=t.dtype, device=t.device).copy_(t.detach().reshape(-1)).view(torch.uint8)
+                for t in (a, b))
+        assert torch.equal(a, b)
+        return
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        same(x, y)
+
+
+def randn(*shape, dtype=torch.bfloat16, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=DEV, dtype=torch.float32).to(dtype)
+
+
+def _layouts(H, T, D, dtype, seed):
+    """[2, H, T, D] tensors of one content type in the layouts a program may hold."""
+    base = randn(2, H, T, D, dtype=dtype, seed=seed)
+    yield "contiguous", base
+    yield "bthd", randn(2, T, H, D, dtype=dtype, seed=seed).transpose(1, 2)
+    yield "wide rows", randn(2, H, T, 2 * D, dtype=dtype, seed=seed)[..., D:]
+    yield "off by one", randn(2 * H * T * D + 1, dtype=dtype, seed=seed)[1:].view(2, H, T, D)
+    yield "d not last", randn(2, H, D, T, dtype=dtype, seed=seed).transpose(2, 3)
+    yield "heads expanded", randn(2, 1, T, D, dtype=dtype, seed=seed).expand(2, H, T, D)
+    yield "odd stride", randn(2, H, T, D + 1, dtype=dtype, seed=seed)[..., :D]
+    yield "order", randn(T, 2, H, D, dtype=dtype, seed=seed).permute(1, 2, 0, 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("D", [8, 20, 64, 100])
+def test_attention_layouts(monkeypatch, dtype, D):
+    T, took = 70, 0
+    for (n1, q), (n2, k) in zip(_layouts(4, T, D, dtype, 1), list(_layouts(2, T, D, dtype, 2))[::-1]):
+        for qq, kk, vv in ((q, k, randn(2, 2, T, D, dtype=dtype, seed=3)), (randn(2, 4, T, D, dtype=dtype, seed=4), k, k)):
+            for kw in ({}, {"window_size": 9}, {"scale": 0.3, "exact_math": True}):
+                def call():
+                    a = [t.detach().requires_grad_(True) for t in (qq, kk, vv)]
+                    o = smooth_attn.sp2norm_flash_attention(*a, **kw)
+                    do = randn(*o.shape, dtype=dtype, seed=5)
+                    return [o, *torch.autograd.grad(o, a, do)]
+                p, n, t = both(monkeypatch, call)
+                same(p, n)
+                took += t
+                same(*both(monkeypatch, lambda: smooth_attn.sp2norm_flash_attention(qq, kk, vv, **kw))[:2])
+    assert took > 0 or D % 8  # some of these forms are ordinary
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("L", [1, 33, 256])
+def test_norm_forms(monkeypatch, dtype, L):
+    fam = smooth_attn.FamilyConfig(alpha=1.5, theta=0.25, power=3)
+    forms = [randn(2, 3, L, L, dtype=dtype), randn(L, L, dtype=dtype), randn(3, L, L, dtype=dtype).transpose(1, 2),
+             randn(2, L, L + 1, dtype=dtype)[..., :L], randn(1, L, L, dtype=dtype).expand(2, L, L)]
+    for x in forms:
+        for kw in ({}, {"family": fam}, {"alpha": 3, "power": 1}):
+            def train():
+                a = x.detach().requires_grad_(True)
+                y = smooth_attn.softplus_norm_causal(a, **kw)
+                (dx,) = torch.autograd.grad(y, a, randn(*y.shape, dtype=dtype, seed=2))
+                return [y, dx]
+            p, n, took = both(monkeypatch, train)
+            same(p, n)
+            assert took == (1 if x.is_contiguous() else 0)
+            for out in (torch.empty_like(x, memory_format=torch.contiguous_format),
+                        torch.empty(*x.shape, 2, device=DEV, dtype=dtype)[..., 0]):
+                p, n, _ = both(monkeypatch, lambda: smooth_attn.softplus_norm_causal_triton_out(out, x, **kw).clone())
+                same(p, n)
+            if x.dim() == 2:
+                p, n, _ = both(monkeypatch, lambda: smooth_attn.softplus_norm_triton(x, **kw))
+                same(p, n)
+
+
+def test_refusals(monkeypatch):
+    x = randn(2, 8, 8)
+    q, k = randn(1, 4, 16, 64), randn(1, 2, 16, 64)
+    calls = [
+        lambda: smooth_attn.softplus_norm_causal(x[:, :4]),
+        lambda: smooth_attn.softplus_norm_causal(x.int()),
+        lambda: smooth_attn.softplus_norm_causal(x.cpu()),
+        lambda: smooth_attn.softplus_norm_causal("x"),
+        lambda: smooth_attn.softplus_norm_causal(randn(1, 1)[:0, :0]),
+        lambda: smooth_attn.softplus_norm_causal_triton_out(x.float(), x),
+        lambda: smooth_attn.softplus_norm_causal_triton_out(x[:1], x),
+        lambda: smooth_attn.softplus_norm_triton_out(x, x),
+        lambda: smooth_attn.softplus_norm_causal(x, family=smooth_attn.FamilyConfig(), alpha=1.0),
+        lambda: smooth_attn.sp2norm_flash_attention(q, k.float(), k),
+        lambda: smooth_attn.sp2norm_flash_attention(q, k, k[:, :1]),
+        lambda: smooth_attn.sp2norm_flash_attention(q[:, :3], k, k),
+        lambda: smooth_attn.sp2norm_flash_attention(q, k.cpu(), k),
+        lambda: smooth_attn.sp2norm_flash_attention(q[0], k, k),
+        lambda: smooth_attn.sp2norm_flash_attention(q, k, k, window_size=-1),
+        lambda: smooth_attn.sp2norm_flash_attention(q, k, k, scale=float("nan")),
+        lambda: smooth_attn.sp2norm_flash_attention(q[:, :, :0], k[:, :, :0], k[:, :, :0]),
+    ]
+    for c in calls:
+        p, n, _ = both(monkeypatch, c)
+        if isinstance(p, Exception):
+            same(p, n)
+            assert str(p) == str(n)
+        else:
+            assert torch.equal(torch.isnan(p), torch.isnan(n)) and torch.equal(p.nan_to_num(), n.nan_to_num())
+
+
+@pytest.mark.parametrize("qd,cd", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                   (torch.float32, torch.float32), (torch.bfloat16, torch.float8_e4m3fn),
+                                   (torch.float32, torch.bfloat16), (torch.float16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("D", [24, 64, 128])
+def test_paged_forms(monkeypatch, qd, cd, D):
+    B, Hkv, P, W = 3, 2, 16, 5
+    table = torch.randperm(B * W, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)).view(B, W)
+    lens = torch.tensor([70, 0, 33], device=DEV)
+    caches = lambda: [randn(B * W, Hkv, P, D, seed=s).to(cd) for s in (2, 3)]
+    forms = [caches(), [c.transpose(1, 2).contiguous().transpose(1, 2) for c in caches()]]
+    if cd != torch.float8_e4m3fn:
+        forms.append([torch.cat([c, c], -1)[..., :D] for c in caches()])
+    for k, v in forms:
+        for t, n in ((table.int(), lens.int()), (table, lens), (table.int().t().contiguous().t(), lens.int()),
+                     (table.int(), torch.stack([lens.int(), lens.int()], 1)[:, 0])):
+            q = randn(B, 4, 1, D, dtype=qd, seed=4)
+            for qq in (q, randn(B, 1, 4, D, dtype=qd, seed=4).transpose(1, 2)):
+                same(*both(monkeypatch, lambda: smooth_attn.sp2norm_paged_attention(qq, k, v, t, n))[:2])
+            for new in (randn(B, Hkv, 2, D, seed=5), randn(B, 2, Hkv, D, seed=5).transpose(1, 2)):
+                def append():
+                    kk, vv = k.clone(memory_format=torch.preserve_format), v.clone(memory_format=torch.preserve_format)
+                    nn = new.to(cd)
+                    return [smooth_attn.sp2norm_paged_kv_append(kk, vv, nn, nn, t, n), kk, vv]
+                same(*both(monkeypatch, append)[:2])
+
+
+def _train(x):
+    y = smooth_attn.softplus_norm_causal(x)
+    return torch.autograd.grad(y, x, torch.ones_like(y))[0]
+
+
+def test_grad_modes_and_parameters(monkeypatch):
+    q, k = randn(1, 4, 40, 64), randn(1, 2, 40, 64)
+    for mode in (torch.no_grad, torch.inference_mode, torch.enable_grad):
+        def call():
+            with mode():
+                a = torch.nn.Parameter(q.clone())
+                o = smooth_attn.sp2norm_flash_attention(a, k, k)
+                y = smooth_attn.softplus_norm_causal(torch.nn.Parameter(q[..., :40].contiguous()))
+                return [o, y]
+        p, n, took = both(monkeypatch, call)
+        same(p, n)
+        assert took == 2
+    # only some inputs need gradients
+    def some():
+        kk = k.clone().requires_grad_(True)
+        return torch.autograd.grad(smooth_attn.sp2norm_flash_attention(q, kk, k), kk, randn(1, 4, 40, 64, seed=3))
+    same(*both(monkeypatch, some)[:2])
+
+
+def test_saved_tensor_hooks_and_checkpoint(monkeypatch):
+    q, k = randn(1, 4, 40, 64), randn(1, 2, 40, 64)
+
+    def hooked():
+        packed = []
+        def pack(t):
+            packed.append(tuple(t.shape))
+            return t.cpu()
+        a, x = q.clone().requires_grad_(True), q[..., :40].clone().requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(DEV)):
+            o = smooth_attn.sp2norm_flash_attention(a, k, k)
+            y = smooth_attn.softplus_norm_causal(x)
+        n = len(packed)
+        g = torch.autograd.grad([o, y], [a, x], [torch.ones_like(o), torch.ones_like(y)])
+        return [torch.tensor(n), *g]
+    same(*both(monkeypatch, hooked)[:2])
+
+    def checkpointed():
+        a = q.clone().requires_grad_(True)
+        o = checkpoint(lambda t: smooth_attn.sp2norm_flash_attention(t, k, k), a, use_reentrant=False)
+        return torch.autograd.grad(o, a, torch.ones_like(o))
+    same(*both(monkeypatch, checkpointed)[:2])
+
+    def changed():  # a saved input changed in place is refused
+        a = q.clone().requires_grad_(True)
+        b = a * 1
+        o = smooth_attn.sp2norm_flash_attention(b, k, k)
+        b.add_(1)
+        return torch.autograd.grad(o, a, torch.ones_like(o))
+    p, n, _ = both(monkeypatch, changed)
+    assert isinstance(p, RuntimeError) and isinstance(n, RuntimeError)
+
+
+def test_transforms_and_subclasses(monkeypatch):
+    x = randn(3, 16, 16)
+    q = randn(2, 2, 16, 32)
+
+    class Sub(torch.Tensor):
+        pass
+
+    def dual():
+        with fwad.dual_level():
+            return smooth_attn.softplus_norm_causal(fwad.make_dual(x, torch.ones_like(x)))
+
+    calls = [
+        lambda: torch.func.vmap(smooth_attn.softplus_norm_causal)(x),
+        lambda: torch.func.vmap(lambda t: smooth_attn.sp2norm_flash_attention(t[None], t[None], t[None]))(q),
+        lambda: torch.func.grad(lambda t: smooth_attn.softplus_norm_causal(t).float().sum())(x),
+        dual,
+    ]
+    for c in calls:
+        p, n, took = both(monkeypatch, c)
+        same(p, n)
+        assert took == 0
+    p, n, took = both(monkeypatch, lambda: smooth_attn.softplus_norm_causal(x.as_subclass(Sub)).as_subclass(torch.Tensor))
+    same(p, n)
+    assert took == 0
+    with torch.device(DEV):  # a function mode
+        p, n, took = both(monkeypatch, lambda: smooth_attn.softplus_norm_causal(x))
+    same(p, n)
+    assert took == 0
+
+    def compiled():
+        torch._dynamo.reset()
+        return torch.compile(lambda t: smooth_attn.softplus_norm_causal(t * 1) + 1, backend="eager")(x)
+    same(*both(monkeypatch, compiled)[:2])
+
+    def double():
+        a = x.clone().requires_grad_(True)
+        y = smooth_attn.softplus_norm_causal(a)
+        (g,) = torch.autograd.grad(y, a, torch.ones_like(y), create_graph=True)
+        return [g]
+    same(*both(monkeypatch, double)[:2])
+
+
+def test_threads_and_streams():
+    xs = [randn(4, 64, 64, seed=s).requires_grad_(True) for s in range(4)]
+    want = [_train(x) for x in xs]
+    got = [None] * 4
+
+    def work(i):
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(s):
+            for _ in range(20):
+                got[i] = _train(xs[i])
+        s.synchronize()
+    torch.cuda.synchronize()
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for a, b in zip(want, got):
+        assert torch.equal(a, b)
