@@ -80,6 +80,7 @@ struct BwdParams {
     // (summed by bwd_split_reduce_kernel); 1 = no split, results stored directly
     int n_split;
     float* part;
+    int dq_groups, kv_groups;  // row groups per block of the two kernels (1 or 2, see merge_groups)
 };
 
 // Plain (cached) 16-byte global load: tiles here are re-read by many blocks.
@@ -110,7 +111,6 @@ struct SwzTile {
     static constexpr int ROWB = D * 2;     // bytes per row
     static constexpr int CPR = D / 8;      // 16-byte chunks per row
     static constexpr int BYTES = 64 * ROWB;
-    static constexpr int NI = 64 * CPR / kBwdThreads;  // DMA loads per lane per tile
     static __device__ __forceinline__ int f(int r) {
         if constexpr (CPR >= 16) return ((r & 3) << 2) | ((r >> 2) & 3);
         else if constexpr (CPR == 8) return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
@@ -136,13 +136,13 @@ __device__ __forceinline__ Vec tr_operand(const unsigned char* p, int lane, int 
 }
 
 // Byte offset (from the tile's first row, row stride rsb) of the source of
-// this lane's DMA load i of a swizzled [64][D] tile: LDS slot s = (4 i +
-// wave) * 64 + lane holds row s / CPR, logical chunk (s % CPR) ^ f(row);
+// this lane's first DMA load of a swizzled [64][D] tile: LDS slot s =
+// wave * 64 + lane holds row s / CPR, logical chunk (s % CPR) ^ f(row);
 // PART: chunks past the head dim dr take kPastTile (zeros).
 template <int D, bool PART>
-__device__ __forceinline__ int swz_src_off(int i, int wave, int lane, int rsb, int dr) {
+__device__ __forceinline__ int swz_src_off(int wave, int lane, int rsb, int dr) {
     using Tl = SwzTile<D>;
-    const int sl = (i * 4 + wave) * 64 + lane;
+    const int sl = wave * 64 + lane;
     const int row = sl / Tl::CPR;
     const int c = (sl - row * Tl::CPR) ^ Tl::f(row);
     if constexpr (!PART) return row * rsb + (c << 4);
@@ -151,24 +151,26 @@ __device__ __forceinline__ int swz_src_off(int i, int wave, int lane, int rsb, i
 
 // Issue the DMA loads of one [64][D] tile whose first row is at `base`
 // (wave-uniform; row stride rsb bytes) into the swizzled LDS tile at `dst`;
-// rows at or past `nrows` read as zeros.  lane_off: swz_src_off(0, ...).
-// Load i covers rows 256/CPR further down than load i - 1 with the same
-// swizzle (f depends on row bits that i does not change), so
-// swz_src_off(i) = i * (256 / CPR) * rsb + swz_src_off(0): each load gets a
-// scalar resource starting i * (256 / CPR) rows in (with the byte count
-// shortened to match, so the zero fill past nrows is unchanged) and one
-// per-lane offset serves them all.
-template <int D>
+// rows at or past `nrows` read as zeros.  lane_off: swz_src_off(...).  The
+// block's NW waves load 64 NW chunks at a time: load i covers rows 64 NW/CPR
+// further down than load i - 1 with the same swizzle (f depends on row bits
+// that i does not change), so each load gets a scalar resource starting
+// i * (64 NW / CPR) rows in (with the byte count shortened to match, so the
+// zero fill past nrows is unchanged) and one per-lane offset serves them all.
+template <int D, int NW>
 __device__ __forceinline__ void issue_swz_tile(const unsigned char* base, int rsb, int nrows, unsigned char* dst,
                                                int wave, int lane_off) {
     using Tl = SwzTile<D>;
-    constexpr int kRowsPerLoad = 256 / Tl::CPR;
+    constexpr int kRowsPerLoad = 64 * NW / Tl::CPR;
+    constexpr int kLoads = (64 * Tl::CPR + 64 * NW - 1) / (64 * NW);  // per lane and tile
+    static_assert(kLoads == 1 || kRowsPerLoad % 16 == 0, "loads of a lane share one swizzle");
     const int nbytes = nrows * rsb;
+    if (kLoads == 1 && wave >= Tl::CPR) return;  // tiles of fewer chunks than lanes
 #pragma unroll
-    for (int i = 0; i < Tl::NI; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
         const int skip = i * kRowsPerLoad * rsb;
         const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base + skip, max(nbytes - skip, 0));
-        tile_dma16(rs, lane_off, dst + (i * 4 + wave) * 64 * 16);
+        tile_dma16(rs, lane_off, dst + (i * NW + wave) * 64 * 16);
     }
 }
 
@@ -182,13 +184,53 @@ __device__ __forceinline__ void weight_and_rr(float s, float sc, float& y, float
     y = sp * sp;
 }
 
+// Key / query split of a block (KS = 2): 8 waves, two for each 32-row tile
+// (slot) of the block's 128 rows; group g = 0, 1 takes the 32-row half g of
+// every staged tile, so a block's walk takes about half the time of a 4-wave
+// block's that handles both halves.  Grids too short to fill the GPU use it
+// (see choose_bwd_plan).  Afterwards each group keeps the 32-column blocks
+// dt = g modulo 2 and adds what the other group has of them, through LDS:
+// slots 0 and 1 in stage array a, 2 and 3 in b, 4 KB per block.  All waves
+// call this; the arrays are free before and after it (barriers inside).
+template <int DT>
+__device__ __forceinline__ void merge_groups(f32x16 (&acc)[DT], int slot, int grp, int lane, unsigned char* a,
+                                             unsigned char* b) {
+    unsigned char* base = (slot < 2 ? a : b) + (slot & 1) * DT * 4096;
+    auto cell = [&](int dt) { return reinterpret_cast<float4*>(base + dt * 4096) + lane; };
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        if (grp != dt % 2) {
+#pragma unroll
+            for (int vg = 0; vg < 4; ++vg)
+                cell(dt)[64 * vg] = float4{acc[dt][vg * 4 + 0], acc[dt][vg * 4 + 1], acc[dt][vg * 4 + 2],
+                                           acc[dt][vg * 4 + 3]};
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        if (grp == dt % 2) {
+#pragma unroll
+            for (int vg = 0; vg < 4; ++vg) {
+                const float4 f = cell(dt)[64 * vg];
+                acc[dt][vg * 4 + 0] += f.x;
+                acc[dt][vg * 4 + 1] += f.y;
+                acc[dt][vg * 4 + 2] += f.z;
+                acc[dt][vg * 4 + 3] += f.w;
+            }
+        }
+    }
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // dQ (and delta)
 // ---------------------------------------------------------------------------
 // PART: the tensors' head dim p.dr is below D (its columns past p.dr read as
 // zeros and are not stored); the kernels with PART false serve dr == D.
-template <typename T, int D, bool EXACT, bool PART>
-__global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams p) {
+// KS: see merge_groups.
+template <typename T, int D, bool EXACT, bool PART, int KS = 1>
+__global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? 2 : 1) void flash_bwd_dq_kernel(BwdParams p) {
     using Ops = MfmaOps<T>;
     using Vec = typename Ops::vec8;
     using Tl = SwzTile<D>;
@@ -202,6 +244,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slot = KS == 1 ? wave : wave & 3, grp = KS == 1 ? 0 : wave >> 2;
     const int hi = lane >> 5;
     const int l32 = lane & 31;
 
@@ -225,7 +268,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
     T* dqp = static_cast<T*>(p.dq) + b * p.dqs[0] + hq * p.dqs[1];
 
     const int q_start = qb * kBwdBQ;
-    const int wq0 = q_start + 32 * wave;
+    const int wq0 = q_start + 32 * slot;
     const int qi = wq0 + l32;
     const int qrow = min(qi, T_ - 1);
 
@@ -246,7 +289,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
     }
     const float dl = dpart + __shfl_xor(dpart, 32);
     const int64_t rbase = static_cast<int64_t>(bh) * T_;
-    if (qi < T_ && hi == 0) p.delta[rbase + qi] = dl;
+    if (qi < T_ && hi == 0 && grp == 0) p.delta[rbase + qi] = dl;
     const float inv_r = 1.f / p.rs[rbase + qrow];
     f32x16 ndl;
 #pragma unroll
@@ -264,8 +307,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
     const float sc = p.scale;
 
     const int ksb = static_cast<int>(p.ks[2] * 2), vsb = static_cast<int>(p.vs[2] * 2);  // row strides (bytes)
-    const int koff = swz_src_off<D, PART>(0, wave, lane, ksb, p.dr);
-    const int voff = swz_src_off<D, PART>(0, wave, lane, vsb, p.dr);
+    const int koff = swz_src_off<D, PART>(wave, lane, ksb, p.dr);
+    const int voff = swz_src_off<D, PART>(wave, lane, vsb, p.dr);
     // Keys past T read as zeros; they only meet masked weights (or rows
     // past T, whose dQ is not written).
     auto stage_base = [&](auto st) -> unsigned char* {
@@ -275,8 +318,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
     auto issue_tile = [&](int j, auto st) {
         const int k0 = j * kBwdKT;
         const int nrows = min(T_ - k0, kBwdKT);
-        issue_swz_tile<D>(kp + static_cast<int64_t>(k0) * ksb, ksb, nrows, stage_base(st), wave, koff);
-        issue_swz_tile<D>(vp + static_cast<int64_t>(k0) * vsb, vsb, nrows, stage_base(st) + Tl::BYTES, wave, voff);
+        issue_swz_tile<D, 4 * KS>(kp + static_cast<int64_t>(k0) * ksb, ksb, nrows, stage_base(st), wave, koff);
+        issue_swz_tile<D, 4 * KS>(vp + static_cast<int64_t>(k0) * vsb, vsb, nrows, stage_base(st) + Tl::BYTES, wave, voff);
     };
 
     // Interior tiles [ja, jb): every row of the wave sees every key (jb: the
@@ -297,7 +340,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
         const unsigned char* Kb = stage_base(st);
         const unsigned char* Vb = stage_base(st) + Tl::BYTES;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
+        for (int kk = 0; kk < 2 / KS; ++kk) {
+            const int kt = KS == 1 ? kk : grp;
             const int kh0 = k0 + kt * 32;
             // the wave's rows see some key of this half
             const bool act = (kh0 <= wq0 + 31) && !(W > 0 && kh0 + 31 <= wq0 - W);
@@ -364,14 +408,16 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
 
     // dS was kept without its per-row factor 2 scale / R_i (applied here).
     // dQ leaves through LDS as whole rows (nontemporal 16-byte chunks).
+    if constexpr (KS == 2) merge_groups<D / 32>(acc, slot, grp, lane, lds0, lds1);
     {
-        constexpr int RB = D * 2 + 16, CPR = D * 2 / 16, RPI = 64 / CPR;
-        static_assert(2 * 32 * RB <= 2 * Tl::BYTES, "two waves' rows per stage array");
+        constexpr int RB = D * 2 + 16, CPR = D * 2 / 16, RPI = 64 / CPR, RPW = 32 / KS;
+        static_assert(2 * 32 * RB <= 2 * Tl::BYTES, "two slots' rows per stage array");
         // both stages are free after the loop's last barrier
-        unsigned char* st = (wave < 2 ? lds0 : lds1) + (wave & 1) * 32 * RB;
+        unsigned char* st = (slot < 2 ? lds0 : lds1) + (slot & 1) * 32 * RB;
         const float f = 2.f * sc * inv_r;
 #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt) {
+            if (KS == 2 && grp != dt % 2) continue;
 #pragma unroll
             for (int vg = 0; vg < 4; ++vg) {
                 const int d0 = dt * 32 + vg * 8 + hi * 4;
@@ -381,12 +427,14 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
                 *reinterpret_cast<uint2*>(st + l32 * RB + d0 * 2) = w;
             }
         }
+        if constexpr (KS == 2) __syncthreads();
 #pragma unroll
-        for (int r0 = 0; r0 < 32; r0 += RPI) {
-            const int r = r0 + lane / CPR, c = lane % CPR;
+        for (int r0 = 0; r0 < RPW; r0 += RPI) {
+            const int rr = r0 + lane / CPR, r = grp * RPW + rr, c = lane % CPR;
             const int qr = wq0 + r;
             const u32x4 v = *reinterpret_cast<const u32x4*>(st + r * RB + c * 16);
-            if (qr < T_ && (!PART || c * 8 < p.dr)) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dqp + qr * p.dqs[2] + c * 8));
+            if (rr < RPW && qr < T_ && (!PART || c * 8 < p.dr))
+                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dqp + qr * p.dqs[2] + c * 8));
         }
     }
 }
@@ -394,8 +442,9 @@ __global__ __launch_bounds__(kBwdThreads, 2) void flash_bwd_dq_kernel(BwdParams 
 // ---------------------------------------------------------------------------
 // dK, dV
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool EXACT, bool PART>
-__global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv_kernel(BwdParams p) {
+// KS: see merge_groups (slots are 32-key tiles, groups take query halves).
+template <typename T, int D, bool EXACT, bool PART, int KS = 1>
+__global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? kBwdDkdvMinBlocks : 1) void flash_bwd_dkdv_kernel(BwdParams p) {
     using Ops = MfmaOps<T>;
     using Vec = typename Ops::vec8;
     using Tl = SwzTile<D>;
@@ -415,14 +464,15 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
     // inside the tile loop, where the wait for it (memory loads complete in
     // order) also waits for the next tile's DMA.  (With fast square roots
     // this leaves no spill; the exact-sqrt build keeps 12 bytes.)
-    constexpr int NXK = D == 128 ? kDkdvLdsK : 0, NXV = D == 128 ? kDkdvLdsV : 0;
-    __shared__ __attribute__((aligned(16))) u32x4 kvx[NXK + NXV > 0 ? NXK + NXV : 1][4][64];  // [K chunks, V chunks][wave][lane]
+    constexpr int NXK = D == 128 ? (KS == 2 ? 5 : kDkdvLdsK) : 0, NXV = D == 128 ? kDkdvLdsV : 0;
+    __shared__ __attribute__((aligned(16))) u32x4 kvx[NXK + NXV > 0 ? NXK + NXV : 1][4 * KS][64];  // [K chunks, V chunks][wave][lane]
     constexpr bool HALFX = D == 128;
-    __shared__ __attribute__((aligned(16))) uint2 kvh[HALFX ? 4 : 1][64];  // [wave][lane]: low 8 bytes of K chunk NXK
+    __shared__ __attribute__((aligned(16))) uint2 kvh[HALFX ? 4 * KS : 1][64];  // [wave][lane]: low 8 bytes of K chunk NXK
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slot = KS == 1 ? wave : wave & 3, grp = KS == 1 ? 0 : wave >> 2;
     const int hi = lane >> 5;
     const int l32 = lane & 31;
 
@@ -456,7 +506,7 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
     T* dvp = static_cast<T*>(p.dv) + b * p.dvs[0] + hk * p.dvs[1];
 
     const int k_start = kb * kBwdBK;
-    const int wk0 = k_start + 32 * wave;
+    const int wk0 = k_start + 32 * slot;
     const int kj = wk0 + l32;
     const int krow = min(kj, T_ - 1);
 
@@ -493,8 +543,8 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
     const float sc = p.scale;
 
     const int qsb = static_cast<int>(p.qs[2] * 2), dsb = static_cast<int>(p.dos[2] * 2);  // row strides (bytes)
-    const int qoff = swz_src_off<D, PART>(0, wave, lane, qsb, p.dr);
-    const int dooff = swz_src_off<D, PART>(0, wave, lane, dsb, p.dr);
+    const int qoff = swz_src_off<D, PART>(wave, lane, qsb, p.dr);
+    const int dooff = swz_src_off<D, PART>(wave, lane, dsb, p.dr);
     float rst = 0.f;
     // Queries past T read as zeros; their weights are masked.
     auto stage_base = [&](auto st) -> unsigned char* {
@@ -511,8 +561,8 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
             reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.dout) + b * p.dos[0] + hq * p.dos[1]));
         const int q0 = qt * kBwdQT;
         const int nrows = min(T_ - q0, kBwdQT);
-        issue_swz_tile<D>(qp + static_cast<int64_t>(q0) * qsb, qsb, nrows, stage_base(st), wave, qoff);
-        issue_swz_tile<D>(dop + static_cast<int64_t>(q0) * dsb, dsb, nrows, stage_base(st) + Tl::BYTES, wave, dooff);
+        issue_swz_tile<D, 4 * KS>(qp + static_cast<int64_t>(q0) * qsb, qsb, nrows, stage_base(st), wave, qoff);
+        issue_swz_tile<D, 4 * KS>(dop + static_cast<int64_t>(q0) * dsb, dsb, nrows, stage_base(st) + Tl::BYTES, wave, dooff);
         // the raw row sum or delta, turned into 1/R or -delta only when it is
         // stored an iteration later, so this load's latency is not waited for here
         // waves 0 and 1 (wave-uniform: the base pointer stays scalar)
@@ -540,7 +590,8 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
         const unsigned char* Qb = stage_base(st);
         const unsigned char* Ob = stage_base(st) + Tl::BYTES;
 #pragma unroll
-        for (int qh = 0; qh < 2; ++qh) {
+        for (int qq = 0; qq < 2 / KS; ++qq) {
+            const int qh = KS == 1 ? qq : grp;
             const int qh0 = q0 + qh * 32;
             // some query of this half sees some key of the wave
             const bool act = (qh0 + 31 >= wk0) && !(W > 0 && qh0 - (wk0 + 31) >= W) && qh0 < T_;
@@ -649,6 +700,10 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
         if (it + 1 < n_it) iteration(it + 1, S1{}, S0{});
     }
 
+    if constexpr (KS == 2) {
+        merge_groups<D / 32>(dkacc, slot, grp, lane, lds0, lds1);
+        merge_groups<D / 32>(dvacc, slot, grp, lane, lds0, lds1);
+    }
     if (n_split > 1) {
         // fp32 partials (zeros for a split without iterations), all D columns
         if (kj < T_) {
@@ -657,6 +712,7 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
             float* pv = pk + bh * T_ * D;
 #pragma unroll
             for (int dt = 0; dt < D / 32; ++dt) {
+                if (KS == 2 && grp != dt % 2) continue;
 #pragma unroll
                 for (int vg = 0; vg < 4; ++vg) {
                     const int d0 = dt * 32 + vg * 8 + hi * 4;
@@ -673,14 +729,16 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
     // dS was kept without its factor 2 scale (1/R_i is already in).  dK and
     // dV leave through LDS as whole rows (nontemporal 16-byte chunks).
     {
-        constexpr int RB = D * 2 + 16, CPR = D * 2 / 16, RPI = 64 / CPR;
-        static_assert(2 * 32 * RB <= 2 * Tl::BYTES, "two waves' rows per stage array");
-        unsigned char* st = (wave < 2 ? lds0 : lds1) + (wave & 1) * 32 * RB;
+        constexpr int RB = D * 2 + 16, CPR = D * 2 / 16, RPI = 64 / CPR, RPW = 32 / KS;
+        static_assert(2 * 32 * RB <= 2 * Tl::BYTES, "two slots' rows per stage array");
+        unsigned char* st = (slot < 2 ? lds0 : lds1) + (slot & 1) * 32 * RB;
         const float f = 2.f * sc;
 #pragma unroll
         for (int which = 0; which < 2; ++which) {
+            if (KS == 2 && which == 1) __syncthreads();  // dK's rows are read
 #pragma unroll
             for (int dt = 0; dt < D / 32; ++dt) {
+                if (KS == 2 && grp != dt % 2) continue;
 #pragma unroll
                 for (int vg = 0; vg < 4; ++vg) {
                     const int d0 = dt * 32 + vg * 8 + hi * 4;
@@ -695,14 +753,15 @@ __global__ __launch_bounds__(kBwdThreads, kBwdDkdvMinBlocks) void flash_bwd_dkdv
                     *reinterpret_cast<uint2*>(st + l32 * RB + d0 * 2) = w;
                 }
             }
+            if constexpr (KS == 2) __syncthreads();
             T* base = which == 0 ? dkp : dvp;
             const int64_t rs = which == 0 ? p.dks[2] : p.dvs[2];
 #pragma unroll
-            for (int r0 = 0; r0 < 32; r0 += RPI) {
-                const int r = r0 + lane / CPR, c = lane % CPR;
+            for (int r0 = 0; r0 < RPW; r0 += RPI) {
+                const int rr = r0 + lane / CPR, r = grp * RPW + rr, c = lane % CPR;
                 const int kr = wk0 + r;
                 const u32x4 v = *reinterpret_cast<const u32x4*>(st + r * RB + c * 16);
-                if (kr < T_ && (!PART || c * 8 < p.dr))
+                if (rr < RPW && kr < T_ && (!PART || c * 8 < p.dr))
                     __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(base + kr * rs + c * 8));
             }
         }
@@ -748,8 +807,14 @@ int launch_bwd_part(const BwdParams& prm, int exact, hipStream_t st) {
         flash_bwd_dq_kernel<T, D, true, PART><<<gq, blk, 0, st>>>(prm);
         flash_bwd_dkdv_kernel<T, D, true, PART><<<gk, blk, 0, st>>>(prm);
     } else {
-        flash_bwd_dq_kernel<T, D, false, PART><<<gq, blk, 0, st>>>(prm);
-        flash_bwd_dkdv_kernel<T, D, false, PART><<<gk, blk, 0, st>>>(prm);
+        if (prm.dq_groups == 2)
+            flash_bwd_dq_kernel<T, D, false, PART, 2><<<gq, dim3(2 * kBwdThreads), 0, st>>>(prm);
+        else
+            flash_bwd_dq_kernel<T, D, false, PART><<<gq, blk, 0, st>>>(prm);
+        if (prm.kv_groups == 2)
+            flash_bwd_dkdv_kernel<T, D, false, PART, 2><<<gk, dim3(2 * kBwdThreads), 0, st>>>(prm);
+        else
+            flash_bwd_dkdv_kernel<T, D, false, PART><<<gk, blk, 0, st>>>(prm);
     }
     if (prm.n_split > 1) {
         const int64_t n_quads = static_cast<int64_t>(prm.B) * prm.Hkv * prm.T * (D / 4);
@@ -794,47 +859,102 @@ int dkdv_iterations(int kb, int T, int G, int W) {
     return G * (qt_end - qt_begin);
 }
 
-// Query-tile splits of the dK/dV blocks.  Causally, key block kb sees the
-// query tiles from its own on, so the first blocks hold the most work; in a
-// grid that does not fill the chip several times over, the GPU idles while
-// they finish.  Splitting every block's iterations n_split ways (fp32
-// partials, summed by one more kernel) shortens that tail at the cost of the
-// partials' traffic.  The count is the one of 1, 2, 4, 8, 16 with the least
-// estimated time: blocks dealt to the XCDs round-robin in the kernel's order
-// (heaviest key blocks first), each XCD running kBwdXcdSlots at once, a block
-// costing its iterations plus two for its set-up and stores, plus a fifth of
-// the longest block for the ragged end, an iteration at 5 us (a 64-query
-// tile of 128 keys with two blocks per CU), and the partials' writes and
-// reads at 5 TB/s; at most 512 MiB of partials.  (Fitted to measured times
-// of shapes from 1 x 2 KV heads x 4096 keys to 2 x 8 x 16384, where it picks
-// the fastest count of each.)  Grids of 4096 blocks or more are not split.
-int dkdv_split_count_uncached(int B, int Hkv, int T, int G, int W, int dr) {
-    const int nkb = (T + kBwdBK - 1) / kBwdBK;
-    const int64_t blocks = static_cast<int64_t>(nkb) * B * Hkv;
-    int best = 1;
-    double best_t = 0.0;
-    for (int S = 1; S <= 16; S *= 2) {
-        // at most 16384 blocks and 512 MiB of partials
-        if (blocks * S > 16384 || bwd_part_bytes(S, B, Hkv, T, dr) > (int64_t(512) << 20)) break;
-        double t = dkdv_split_makespan(nkb, B * Hkv, S, kBwdXcdSlots, 2.0,
-                                       [&](int kb) { return dkdv_iterations(kb, T, G, W); }) *
-                   5.0;  // us
-        // the partials written, then read by the sum kernel
-        if (S > 1) t += 2.0 * static_cast<double>(bwd_part_bytes(S, B, Hkv, T, dr)) / 5e6 + 5.0;
-        if (S == 1 || t < best_t) {
-            best = S;
-            best_t = t;
+// How a backward's two kernels share out their work.
+//
+// Causally, key block kb sees the query tiles from its own on and query block
+// qb the key tiles up to its own, so the first dK/dV and the last dQ blocks
+// hold the most work; in a grid that does not fill the chip several times
+// over, the GPU idles while they finish.  Two things shorten them:
+//  * groups = 2: blocks of 8 waves, each wave walking one half of every tile
+//    (merge_groups), merged in LDS;
+//  * S > 1 (dK/dV): every block's iterations split S ways, fp32 partials
+//    summed by one more kernel.
+// Each candidate is estimated as the longer of the longest block and all
+// work shared out evenly, plus a quarter of the other (the ragged end), plus
+// the partials' traffic; constants in us, fitted to 83 measured shapes (bf16,
+// D = 64 and 128, T = 128 .. 8192, 8 to 64 heads, GQA 1, 4 and 8, windows 0
+// to 1024), on which the choice averages 0.4% over the fastest candidate
+// and is at worst 6% over it.  dQ + dK/dV, one group and the S of an
+// earlier rule -> this choice: [4,12,1024,64] 68 -> 55 us, [1,32,1024,128]
+// 91 -> 73, [1,32,2048,128] 195 -> 162, [2,32/8,3000,128] window 1024 (S = 4
+// -> 1) 419 -> 382, [1,32/8,2048,128] 199 -> 168; full grids keep one group.
+struct BwdCosts {
+    double dq_setup[2], dq_tile[2], dq_share[2];  // by groups - 1: block setup, a tile of the longest block, a tile's share of a CU
+    double kv_setup, kv_iter[2], kv_share[2], kv_share_setup, part_tb_s, part_setup;
+};
+constexpr BwdCosts kBwdCosts128 = {{4.1, 12.7}, {3.2, 1.08}, {0.74, 0.87}, 21.7, {3.47, 3.22}, {3.16, 3.13}, 5.2, 6.0, 10.0};
+constexpr BwdCosts kBwdCosts64 = {{6.8, 9.7}, {2.3, 1.66}, {1.35, 1.78}, 7.5, {2.81, 2.40}, {1.67, 1.94}, 4.3, 3.6, 5.3};
+
+struct BwdPlan {
+    int dq_groups = 1, kv_groups = 1, n_split = 1;
+};
+
+double with_ragged_end(double longest, double shared) {
+    return std::max(longest, shared) + 0.25 * std::min(longest, shared);
+}
+
+// max_split: the most splits the caller's workspace holds; groups: whether
+// blocks of two groups may be used (exact square roots have none).
+BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, int max_split, bool groups) {
+    constexpr double kCus = 256.0;
+    const BwdCosts& c = bwd_kernel_d(dr) == 128 ? kBwdCosts128 : kBwdCosts64;
+    const int nkb = (T + kBwdBK - 1) / kBwdBK, nqb = (T + kBwdBQ - 1) / kBwdBQ;
+    const int n_kv = (T + kBwdKT - 1) / kBwdKT;
+    int64_t kv_sum = 0, dq_sum = 0;
+    int kv_max = 0, dq_max = 0;
+    for (int kb = 0; kb < nkb; ++kb) {
+        const int n = dkdv_iterations(kb, T, G, W);
+        kv_sum += n;
+        kv_max = std::max(kv_max, n);
+    }
+    for (int qb = 0; qb < nqb; ++qb) {
+        const int q0 = qb * kBwdBQ;
+        const int n = std::min((q0 + kBwdBQ + kBwdKT - 1) / kBwdKT, n_kv) -
+                      (W > 0 ? std::max(0, q0 - W + 1) / kBwdKT : 0);
+        dq_sum += n;
+        dq_max = std::max(dq_max, n);
+    }
+    const double kv_heads = static_cast<double>(B) * Hkv;
+    BwdPlan best;
+    double dq_t = 0.0, kv_t = 0.0;
+    for (int g = 0; g < (groups ? 2 : 1); ++g) {
+        const double t = with_ragged_end(
+            c.dq_setup[g] + dq_max * c.dq_tile[g],
+            kv_heads * G * (0.5 * nqb * c.dq_setup[g] + static_cast<double>(dq_sum) * c.dq_share[g]) / kCus);
+        if (g == 0 || t < 0.98 * dq_t) {
+            best.dq_groups = g + 1;
+            dq_t = t;
+        }
+        for (int S = 1; S <= max_split; S *= 2) {
+            const int64_t bytes = bwd_part_bytes(S, B, Hkv, T, dr);
+            // an iteration of the longest block each, at most 16384 blocks and 512 MiB of partials
+            if (S > 1 && (S > kv_max || static_cast<int64_t>(nkb) * B * Hkv * S > 16384 || bytes > (int64_t(512) << 20))) break;
+            double u = with_ragged_end(
+                c.kv_setup + (kv_max + S - 1) / S * c.kv_iter[g],
+                kv_heads * (nkb * S * (g + 1) * c.kv_share_setup + static_cast<double>(kv_sum) * c.kv_share[g]) / kCus);
+            // the partials written, then read by the sum kernel
+            if (S > 1) u += c.part_setup + 2.0 * static_cast<double>(bytes) / (c.part_tb_s * 1e6);
+            if ((g == 0 && S == 1) || u < kv_t) {
+                best.kv_groups = g + 1;
+                best.n_split = S;
+                kv_t = u;
+            }
         }
     }
     return best;
 }
 
-int dkdv_split_count(int B, int Hkv, int T, int G, int W, int dr) {
+constexpr int kMaxSplit = 16;
+BwdPlan choose_bwd_plan(int B, int Hkv, int T, int G, int W, int dr, int max_split, bool groups) {
     const int64_t blocks = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv;
-    if (blocks >= 8 * kBwdXcdSlots * 8 || blocks == 0) return 1;
-    static SplitCountCache cache;
-    const int key[6] = {B, Hkv, T, G, W, bwd_kernel_d(dr)};
-    return cache.get(key, [&] { return dkdv_split_count_uncached(B, Hkv, T, G, W, dr); });
+    if (blocks >= 8 * kBwdXcdSlots * 8 || blocks == 0) return BwdPlan{};  // full grids
+    static SplitCountCache cache;  // (a plan is kept as one number)
+    const int key[6] = {B, Hkv, T, G, W, (bwd_kernel_d(dr) << 8) | (max_split << 1) | (groups ? 1 : 0)};
+    const int code = cache.get(key, [&] {
+        const BwdPlan p = choose_bwd_plan_uncached(B, Hkv, T, G, W, dr, max_split, groups);
+        return (p.n_split << 4) | (p.kv_groups << 2) | p.dq_groups;
+    });
+    return BwdPlan{code & 3, (code >> 2) & 3, code >> 4};
 }
 
 }  // namespace
@@ -846,7 +966,11 @@ extern "C" int64_t sa_flash_bwd_workspace_size(int B, int Hq, int Hkv, int T, in
     if (dtype != SA_BF16 && dtype != SA_F16) return 0;
     if (B == 0 || T == 0 || D > 512) return 0;
     if (D > 128) return flash_bwd_wide_workspace_size(B, Hq, Hkv, T, D, window_size);
-    return bwd_part_bytes(dkdv_split_count(B, Hkv, T, Hq / Hkv, window_size, D), B, Hkv, T, D);
+    const int n_split = choose_bwd_plan(B, Hkv, T, Hq / Hkv, window_size, D, kMaxSplit, true).n_split;
+    // room for two splits in the smallest grids, also where none is chosen
+    // (exact square roots, which have no groups, may then split)
+    const bool small = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv < 64;
+    return bwd_part_bytes(small ? std::max(n_split, 2) : n_split, B, Hkv, T, D);
 }
 
 extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -916,17 +1040,18 @@ extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, cons
     prm.window = window_size;
     prm.dr = D;
     prm.scale = scale;
-    // the library's split count, or the largest power of two below it whose
-    // partials fit the workspace
-    prm.n_split = 1;
-    prm.part = nullptr;
+    // the plan among the split counts whose partials fit the workspace
+    int max_split = 1;
     if (workspace && workspace_bytes > 0) {
         if (!aligned16(workspace)) return SA_ERR_BAD_STRIDE;
-        int ns = dkdv_split_count(B, Hkv, T, prm.G, window_size, D);
-        while (ns > 1 && bwd_part_bytes(ns, B, Hkv, T, D) > workspace_bytes) ns /= 2;
-        prm.n_split = ns;
-        prm.part = static_cast<float*>(workspace);
+        max_split = kMaxSplit;
+        while (max_split > 1 && bwd_part_bytes(max_split, B, Hkv, T, D) > workspace_bytes) max_split /= 2;
     }
+    const BwdPlan plan = choose_bwd_plan(B, Hkv, T, prm.G, window_size, D, max_split, !exact_math);
+    prm.n_split = plan.n_split;
+    prm.part = plan.n_split > 1 ? static_cast<float*>(workspace) : nullptr;
+    prm.dq_groups = plan.dq_groups;
+    prm.kv_groups = plan.kv_groups;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int ex = exact_math ? 1 : 0;
     if (dtype == SA_BF16) return launch_bwd_d<bf16>(prm, ex, s);
