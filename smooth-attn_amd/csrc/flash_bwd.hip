@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? 2 : 1) void flash_bwd_d
 
     const int nqb = (p.T + kBwdBQ - 1) / kBwdBQ;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, kBwdXcdSlots, step, unit, sub);
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, kBwdXcdSlots, true, step, unit, sub);
     const int qb = nqb - 1 - step;  // heaviest (latest) query blocks first
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? kBwdDkdvMinBlocks : 1) 
     }
     int kb, unit, sub;
     // earliest key blocks see the most queries: first
-    grouped_block(ob, p.B * p.Hkv, 1, nkb, kBwdXcdSlots, kb, unit, sub);
+    grouped_block(ob, p.B * p.Hkv, 1, nkb, kBwdXcdSlots, true, kb, unit, sub);
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
     const int T_ = p.T;
@@ -870,27 +870,33 @@ int dkdv_iterations(int kb, int T, int G, int W) {
 //  * S > 1 (dK/dV): every block's iterations split S ways, fp32 partials
 //    summed by one more kernel.
 // Each candidate is estimated as the longer of the longest block and all
-// work shared out evenly, plus a quarter of the other (the ragged end), plus
-// the partials' traffic; constants in us, fitted to 83 measured shapes (bf16,
-// D = 64 and 128, T = 128 .. 8192, 8 to 64 heads, GQA 1, 4 and 8, windows 0
-// to 1024), on which the choice averages 0.4% over the fastest candidate
-// and is at worst 6% over it.  dQ + dK/dV, one group and the S of an
-// earlier rule -> this choice: [4,12,1024,64] 68 -> 55 us, [1,32,1024,128]
-// 91 -> 73, [1,32,2048,128] 195 -> 162, [2,32/8,3000,128] window 1024 (S = 4
-// -> 1) 419 -> 382, [1,32/8,2048,128] 199 -> 168; full grids keep one group.
+// work shared out evenly, plus a part of the other (the ragged end), plus the
+// partials' traffic; constants in us, fitted to 430 measured shapes (bf16,
+// D = 64 to 128, T = 256 .. 8192, up to 1100 blocks of 256 rows, GQA 1 to 8,
+// windows of none to half), on which the choice averages 0.3% over the
+// fastest candidate and is at worst 7% over it.  dQ + dK/dV, one group and
+// the S of an earlier rule -> two groups or another S: [4,12,1024,64] 68 ->
+// 55 us, [1,32,1024,128] 91 -> 73, [1,32,2048,128] 195 -> 162,
+// [2,32/8,3000,128] window 1024 (S = 4 -> 1) 419 -> 382, [1,32/8,2048,128] 199
+// -> 168; full grids keep one group.
 struct BwdCosts {
-    double dq_setup[2], dq_tile[2], dq_share[2];  // by groups - 1: block setup, a tile of the longest block, a tile's share of a CU
-    double kv_setup, kv_iter[2], kv_share[2], kv_share_setup, part_tb_s, part_setup;
+    // by groups - 1: setup and tile of the longest block, the same of a block in a full grid (per CU);
+    // *_alone: a tile of a one-group block that has its CU to itself
+    double dq_setup[2], dq_alone, dq_tile[2], dq_share_setup[2], dq_share[2], dq_ragged;
+    double kv_setup, kv_alone, kv_iter[2], kv_share_setup[2], kv_share[2], kv_ragged;
+    double part_tb_s, part_setup;
 };
-constexpr BwdCosts kBwdCosts128 = {{4.1, 12.7}, {3.2, 1.08}, {0.74, 0.87}, 21.7, {3.47, 3.22}, {3.16, 3.13}, 5.2, 6.0, 10.0};
-constexpr BwdCosts kBwdCosts64 = {{6.8, 9.7}, {2.3, 1.66}, {1.35, 1.78}, 7.5, {2.81, 2.40}, {1.67, 1.94}, 4.3, 3.6, 5.3};
+constexpr BwdCosts kBwdCosts128 = {{3.5, 10.7}, 2.14, {2.43, 0.89}, {6.8, 5.7}, {0.43, 1.74}, 0.41,
+                                   6.4, 2.79, {3.33, 2.72}, {7.0, 9.9}, {1.85, 2.53}, 0.05, 8.0, 14.3};
+constexpr BwdCosts kBwdCosts64 = {{3.7, 10.5}, 2.02, {1.88, 0.96}, {5.7, 8.0}, {1.06, 1.63}, 0.09,
+                                  12.5, 2.59, {2.59, 1.54}, {3.3, 10.2}, {1.59, 2.42}, 0.38, 5.0, 4.2};
 
 struct BwdPlan {
     int dq_groups = 1, kv_groups = 1, n_split = 1;
 };
 
-double with_ragged_end(double longest, double shared) {
-    return std::max(longest, shared) + 0.25 * std::min(longest, shared);
+double with_ragged_end(double longest, double shared, double ragged) {
+    return std::max(longest, shared) + ragged * std::min(longest, shared);
 }
 
 // max_split: the most splits the caller's workspace holds; groups: whether
@@ -915,23 +921,36 @@ BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, in
         dq_max = std::max(dq_max, n);
     }
     const double kv_heads = static_cast<double>(B) * Hkv;
+    // a tile's time in a grid of `blocks` blocks: alone on the CU up to one block per CU, shared from two on
+    const auto tile_time = [](double alone, double shared, double blocks) {
+        return alone + (shared - alone) * std::min(1.0, std::max(0.0, blocks / kCus - 1.0));
+    };
+    // Under a window of up to half the rows the blocks are nearly equal; where
+    // all run at once on most of the slots (D = 128: two blocks per CU) neither
+    // shortens the whole ([2,32/8,3000] window 1024: S = 1 / 2 / 4, two groups
+    // 382 / 411 / 419, 442 us).
+    if (W > 0 && 2 * W <= T && bwd_kernel_d(dr) == 128 && nkb * kv_heads > 1.25 * kCus && nkb * kv_heads <= 2 * kCus)
+        max_split = 0;
     BwdPlan best;
     double dq_t = 0.0, kv_t = 0.0;
     for (int g = 0; g < (groups ? 2 : 1); ++g) {
         const double t = with_ragged_end(
-            c.dq_setup[g] + dq_max * c.dq_tile[g],
-            kv_heads * G * (0.5 * nqb * c.dq_setup[g] + static_cast<double>(dq_sum) * c.dq_share[g]) / kCus);
+            c.dq_setup[g] + dq_max * (g == 0 ? tile_time(c.dq_alone, c.dq_tile[0], nqb * kv_heads * G) : c.dq_tile[1]),
+            kv_heads * G * (nqb * c.dq_share_setup[g] + static_cast<double>(dq_sum) * c.dq_share[g]) / kCus, c.dq_ragged);
         if (g == 0 || t < 0.98 * dq_t) {
             best.dq_groups = g + 1;
             dq_t = t;
         }
+        if (g == 1 && kv_max < 4) break;  // nothing to share
         for (int S = 1; S <= max_split; S *= 2) {
             const int64_t bytes = bwd_part_bytes(S, B, Hkv, T, dr);
             // an iteration of the longest block each, at most 16384 blocks and 512 MiB of partials
             if (S > 1 && (S > kv_max || static_cast<int64_t>(nkb) * B * Hkv * S > 16384 || bytes > (int64_t(512) << 20))) break;
             double u = with_ragged_end(
-                c.kv_setup + (kv_max + S - 1) / S * c.kv_iter[g],
-                kv_heads * (nkb * S * (g + 1) * c.kv_share_setup + static_cast<double>(kv_sum) * c.kv_share[g]) / kCus);
+                c.kv_setup + (kv_max + S - 1) / S * (g == 0 ? tile_time(c.kv_alone, c.kv_iter[0], nkb * kv_heads * S)
+                                                            : c.kv_iter[1]),
+                kv_heads * (nkb * S * c.kv_share_setup[g] + static_cast<double>(kv_sum) * c.kv_share[g]) / kCus,
+                c.kv_ragged);
             // the partials written, then read by the sum kernel
             if (S > 1) u += c.part_setup + 2.0 * static_cast<double>(bytes) / (c.part_tb_s * 1e6);
             if ((g == 0 && S == 1) || u < kv_t) {

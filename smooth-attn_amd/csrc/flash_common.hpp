@@ -83,13 +83,27 @@ __device__ __forceinline__ V lds_read_tr16_pair(const void* p0, const void* p1) 
 // fastest, so the blocks in flight share a handful of K/V (or Q/dO) streams
 // and the group's heavy steps still start early.  Otherwise step-major over
 // all (unit, sub).
+//
+// `uneven` (steps differ in work): where a group's blocks are no multiple of
+// xcd_slots, the next group's heavy steps start late and the last group's end
+// late, up to half again the balanced time in grids of a few rounds.  Up to
+// kOneGroupRounds blocks per slot an XCD then takes all its units as one
+// group, heavy steps first throughout (as groups -> as one; bf16, D = 128,
+// forward / backward us: [1,32,3000] 126 / 397 -> 102 / 341, [2,32,1536] 71 /
+// 227 -> 58 / 193, [4,32,3000], 6 rounds, 400 / 1236 -> 374 / 1152).  Longer
+// grids lose more L2 hits than they gain ([4,32,5000], 10 rounds, 931 / 3022
+// -> 934 / 3080), and so do equal steps ([2,32/8,3000] window 1024 forward 122
+// -> 125).
+constexpr int kOneGroupRounds = 8;
 __device__ __forceinline__ void grouped_block(int id, int n_units, int n_sub, int n_steps, int xcd_slots,
-                                              int& step, int& unit, int& sub) {
+                                              bool uneven, int& step, int& unit, int& sub) {
     if ((n_units & 7) == 0) {
         const int x = id & 7;
         const int j = id >> 3;
         const int nh = (n_units >> 3) * n_sub;  // (unit, sub) pairs on this XCD
-        const int gu = min(max(1, (xcd_slots + n_sub * n_steps - 1) / (n_sub * n_steps)), n_units >> 3);
+        int gu = min(max(1, (xcd_slots + n_sub * n_steps - 1) / (n_sub * n_steps)), n_units >> 3);
+        if (uneven && nh * n_steps <= kOneGroupRounds * xcd_slots && gu * n_sub * n_steps % xcd_slots != 0)
+            gu = n_units >> 3;
         const int gh = gu * n_sub;  // pairs per group
         const int grp = j / (gh * n_steps);
         const int r = j - grp * (gh * n_steps);

@@ -100,10 +100,18 @@ __global__ __launch_bounds__(256) void rope_rotate_any(const T* __restrict__ x, 
 }
 
 // Estimated microseconds of the forward with key split KS, one block per CU:
-// the longest block, or all blocks shared out evenly.  A block costs `setup`
-// (loads of Q and the first tile, the epilogue) and `tile` per K/V tile.
+// the longer of the longest block and all blocks shared out evenly, plus a
+// part of the other (the ragged end).
+struct SplitCosts {
+    double setup, tile;        // the longest block: loads of Q and the first tile and the epilogue; per K/V tile
+    double share_setup, share; // the same of a block in a full grid, per CU
+};
+struct ForwardCosts {
+    SplitCosts ks1, ks2, ks4;
+    double ragged, margin;
+};
 template <int KS>
-double forward_estimate(const FlashParams& p, double setup, double tile) {
+double forward_estimate(const FlashParams& p, const SplitCosts& c, double ragged) {
     constexpr int kCus = 256;
     constexpr int BQ = Split<KS>::BQ, BKV = Split<KS>::BKV;
     const int nqb = (p.T + BQ - 1) / BQ, n_kv = (p.T + BKV - 1) / BKV;
@@ -116,29 +124,38 @@ double forward_estimate(const FlashParams& p, double setup, double tile) {
         sum += n;
         longest = std::max(longest, n);
     }
-    const double all = static_cast<double>(p.B) * p.Hq * (nqb * setup + static_cast<double>(sum) * tile);
-    return std::max(setup + longest * tile, all / kCus);
+    const double one = c.setup + longest * c.tile;
+    const double all = static_cast<double>(p.B) * p.Hq * (nqb * c.share_setup + static_cast<double>(sum) * c.share) / kCus;
+    return std::max(one, all) + ragged * std::min(one, all);
 }
 
 // Key split of a launch (1, 2 or 4).  A split shortens the blocks, for grids
 // that leave CUs idle or waiting for the longest block, but costs a merge and
-// more barriers per MFMA, so full grids keep KS = 1.  The constants are fitted
-// to 76 shapes (bf16, D = 64 and 128, T = 128 .. 8192, 8 to 64 heads, windows
-// 0 to 1024); the choice is within 7% of the fastest on all of them.  KS = 1 /
-// 2 / 4 in us, D = 128: [1,32/8,512] 18.7 / 15.3 / 13.1, [1,32/8,1024] 31.4 /
-// 23.4 / 26.2, [1,32/8,2048] 58.0 / 52.4 / 69.9, [1,8,2048] 54.3 / 35.5 / 25.6,
-// [2,32/8,1024] 34.0 / 35.3 / 49.4.  Grids of over 512 blocks never gained
-// more than their noise and skip the estimate.  KS = 4 walks tiles of 128
-// rows, whose 32-bit offsets bound the row stride.
+// more barriers per MFMA, so full grids keep KS = 1 at D = 128; at D = 64 two
+// KS = 2 blocks fit a CU (under 128 registers) and it wins over most sizes.
+// The constants (us) are fitted to 430 measured shapes (bf16, T = 256 ..
+// 8192, up to 1100 blocks of 256 rows, GQA 1 to 8, windows of none to half),
+// on which the choice averages 0.3% over the fastest KS.  KS = 1 / 2 / 4 in us,
+// D = 128: [1,32/8,512] 18.7 / 15.3 / 13.1, [1,32/8,1024] 31.4 / 23.4 / 26.2,
+// [1,32/8,2048] 58.0 / 52.4 / 69.9, [1,8,2048] 54.3 / 35.5 / 25.6,
+// [2,32/8,1024] 34.0 / 35.3 / 49.4; D = 64: [1,32/8,5760] 207 / 179 / 251.
+// Longer grids (over 512 blocks of 256 rows, 768 at D = 64) gain no more than
+// their noise or lose ([1,32,8128] at D = 64, 1024 blocks, 350 / 374) and skip
+// the estimate.  KS = 4 walks tiles of 128 rows, whose 32-bit offsets bound
+// the row stride.
+constexpr ForwardCosts kForwardCosts128 = {{3.4, 2.35, 3.9, 2.99}, {6.3, 0.84, 7.5, 1.31}, {6.8, 1.16, 7.4, 1.20}, 0.03, 0.78};
+constexpr ForwardCosts kForwardCosts64 = {{9.7, 1.99, 4.6, 3.53}, {8.3, 0.85, 3.3, 1.25}, {7.1, 1.35, 8.1, 1.15}, 0.35, 1.02};
 int key_split_for(const FlashParams& p, int qk_bytes, int v_bytes) {
-    if (static_cast<int64_t>(p.nqb) * p.B * p.Hq > 512) return 1;
+    const int64_t limit = p.dr > 32 && p.dr <= 64 ? 768 : 512;
+    if (static_cast<int64_t>(p.nqb) * p.B * p.Hq > limit) return 1;
     constexpr int64_t kMaxStride4 = int64_t(1) << 23;
-    const double e1 = forward_estimate<1>(p, 5.0, 1.75);
-    const double e2 = forward_estimate<2>(p, 8.0, 0.95);
+    const ForwardCosts& c = p.dr > 64 ? kForwardCosts128 : kForwardCosts64;
+    const double e1 = forward_estimate<1>(p, c.ks1, c.ragged);
+    const double e2 = forward_estimate<2>(p, c.ks2, c.ragged);
     const double e4 = p.ks[2] * qk_bytes <= kMaxStride4 && p.vs[2] * v_bytes <= kMaxStride4
-                          ? forward_estimate<4>(p, 7.0, 1.4)
-                          : e2;
-    if (std::min(e2, e4) > 0.97 * e1) return 1;
+                          ? forward_estimate<4>(p, c.ks4, c.ragged)
+                          : 2.0 * e2;
+    if (std::min(e2, e4) >= c.margin * e1) return 1;
     return e4 < e2 ? 4 : 2;
 }
 

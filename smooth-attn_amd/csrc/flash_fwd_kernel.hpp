@@ -147,7 +147,11 @@ __device__ __forceinline__ u32x4 tile_load16(const T* p) {
 constexpr int kBlocksPerXcd = 32;
 __device__ __forceinline__ void block_coords(const FlashParams& p, int& qb, int& b, int& hq) {
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, p.nqb, kBlocksPerXcd, step, unit, sub);
+    // (under a window of up to half the rows most query blocks walk equally
+    // many tiles; and groups of one KV head that fill the XCD by themselves
+    // are balanced within 5%, where the L2 hits count more)
+    const bool uneven = (p.window <= 0 || 2 * p.window > p.T) && p.G * p.nqb <= kBlocksPerXcd;
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, p.nqb, kBlocksPerXcd, uneven, step, unit, sub);
     qb = p.nqb - 1 - step;
     b = unit / p.Hkv;
     hq = (unit - b * p.Hkv) * p.G + sub;
@@ -165,9 +169,10 @@ __device__ __forceinline__ void block_coords(const FlashParams& p, int& qb, int&
 // across the tile boundary).  Squareplus needs no maximum, so the groups'
 // unnormalised O and row sums are just added, through LDS after the last
 // tile, in the order of the groups: no workspace, no second kernel, and
-// results that do not depend on timing.
+// results that do not depend on timing.  At D = 64 KS = 2 needs under 128
+// registers and is held to that, so two blocks fit a CU.
 template <typename T, int D, bool QK8, bool V8, bool EXACT, bool ROPE, bool FOLD = false, int KS = 1>
-__global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashParams p) {
+__global__ __launch_bounds__(kThreads, KS == 2 && D == 64 ? 4 : 1) void flash_fwd_kernel(FlashParams p) {
     using Gm = Geom<T, D, QK8, V8, KS>;
     constexpr int kBKV = Split<KS>::BKV, kStages = Split<KS>::STAGES;
     constexpr int QW = Split<KS>::QW, kBQ2 = Split<KS>::BQ;
