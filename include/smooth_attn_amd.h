@@ -242,6 +242,18 @@ int sa_fp8_quantize(const void* x, void* x8, int64_t n, int dtype,
                     float* amax_ws, float* scale_out, sa_stream_t stream);
 
 /*
+ * The same of 1 to 4 tensors of one dtype, each with a scale of its own, in
+ * two launches over all of them: x[i] (n[i] contiguous elements) -> x8[i] and
+ * scales_out[i].  x, x8 and n are host arrays of count entries.  amax_ws:
+ * count * SA_FP8_AMAX_WORDS fp32 of workspace, contents ignored.  Codes and
+ * scales are those of sa_fp8_quantize.
+ */
+#define SA_FP8_AMAX_WORDS 1024
+int sa_fp8_quantize_many(int count, const void* const* x, void* const* x8,
+                         const int64_t* n, int dtype, float* amax_ws,
+                         float* scales_out, sa_stream_t stream);
+
+/*
  * fp8 fused causal attention forward.  q8, k8: float8_e4m3fn; v: e4m3fn
  * (v_dtype SA_FP8_E4M3FN, as the reference entry point quantises V) or bf16
  * (v_dtype SA_BF16).  Scales are device pointers to one fp32 each (v_scale

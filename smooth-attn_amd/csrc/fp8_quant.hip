@@ -1,26 +1,53 @@
 // Per-tensor absmax quantisation to float8_e4m3fn, entirely on the device
 // (reference kernels.py:2592-2601, which synchronises through .item()):
 //   scale = max(amax|x| / 448, 1e-12);  x8 = e4m3fn(clamp(x / scale, +-448))
-// Three launches on one stream: zero the amax word, reduce amax with one
-// atomicMax per block (non-negative floats order like their bit patterns),
-// then quantise.  x / scale is a true division so the codes match torch's
-// fp32 division followed by the round-to-nearest-even e4m3fn cast.  Both
-// passes read 16 bytes per lane and load when x is 16-byte aligned (the
-// remainder, and unaligned inputs, element by element), several loads in
-// flight per lane.
+// Both entry points run the same two passes.  The first leaves one maximum
+// per block; the second reduces a tensor's maxima in every block and writes
+// the codes.  sa_fp8_quantize_many puts up to kMaxTensors tensors into each
+// pass, its blocks dealt out by size: a forward from 16-bit q, k and v takes
+// two launches where a call per tensor takes nine (three each, the first to
+// clear the one word that its blocks meet in).
+// HBM binds the large sizes and the launches the small ones: q, k and v of a
+// [2,32/8,8192,128] forward 107 -> 86 us (31.5 us at 6.4 TB/s, then 54 us at
+// 5.6 TB/s), its whole call 945 -> 922 us; a [1,32/8,2048,128] call
+// 83 -> 63 us.  Walking the second pass backwards, towards what the first
+// read last, changed nothing.  Both passes
+// read 16 bytes per lane and load when x is 16-byte aligned (the remainder,
+// and unaligned inputs, element by element), several loads in flight per lane.
 #include "common.hpp"
 
 namespace sa {
 namespace {
 
 constexpr int kQThreads = 256;
-// The amax pass ends in one same-address atomicMax per block; those
-// serialise, so the pass runs on at most kAmaxBlocks blocks (one per CU)
-// with kAmaxUnroll loads in flight per lane (measured on config 4's Q,
-// 67M bf16: 4096 blocks 95 us, 512 blocks 64 us, 256 blocks x 8 loads 62 us
-// for amax + quantise together).
-constexpr unsigned kAmaxBlocks = 256;
+constexpr int kMaxTensors = 4;
+// Maxima kept per tensor, so also the most blocks of the amax pass on one:
+// four per CU over all tensors.  A caller that brings one word instead of
+// kSlots has the blocks meet in it by atomicMax (non-negative floats order
+// like their bit patterns); those serialise, so that route keeps to one block
+// per CU (67M bf16: 4096 blocks 95 us, 512 blocks 64 us, 256 blocks x 8 loads
+// 62 us for both passes).
+constexpr unsigned kSlots = SA_FP8_AMAX_WORDS;
+constexpr unsigned kAmaxAtomicBlocks = 256;
 constexpr int kAmaxUnroll = 8;
+constexpr unsigned kQuantBlocks = 4096;
+
+struct QuantTensor {
+    const void* x;
+    uint8_t* x8;
+    int64_t n;
+    uint32_t* maxima;  // bits of the blocks' maxima
+    float* scale_out;
+    unsigned amax_begin, amax_blocks;    // this tensor's blocks of the amax pass
+    unsigned quant_begin, quant_blocks;  // and of the second
+    int vec;                             // 16-byte loads
+};
+
+struct QuantArgs {
+    QuantTensor t[kMaxTensors];
+    int count;
+    int shared_word;  // the maxima are one word, met by atomicMax
+};
 
 __global__ void fill_zero_u32(uint32_t* p) { p[0] = 0u; }
 
@@ -33,18 +60,34 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kQThreads) void amax_kernel(const T* __restrict__ x, int64_t n, uint32_t* amax_bits,
-                                                         int vec) {
-    constexpr int NV = 16 / sizeof(T);  // elements per 16-byte load
+// The largest v of the block, in every thread.
+__device__ __forceinline__ float block_max(float v) {
     __shared__ float part[kQThreads / 64];
+    v = wave_max(v);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float b = part[0];
+#pragma unroll
+    for (int w = 1; w < kQThreads / 64; ++w) b = fmaxf(b, part[w]);
+    return b;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
+    int ti = 0;
+    while (ti + 1 < a.count && blockIdx.x >= a.t[ti + 1].amax_begin) ++ti;
+    const QuantTensor& qt = a.t[ti];
+    const T* __restrict__ x = static_cast<const T*>(qt.x);
+    const int64_t n = qt.n;
+    const unsigned block = blockIdx.x - qt.amax_begin;
+    constexpr int NV = 16 / sizeof(T);  // elements per 16-byte load
     float m = 0.f;
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kQThreads;
-    const int64_t tid0 = static_cast<int64_t>(blockIdx.x) * kQThreads + threadIdx.x;
-    const int64_t nv = vec ? n / NV : 0;
+    const int64_t stride = static_cast<int64_t>(qt.amax_blocks) * kQThreads;
+    const int64_t tid0 = static_cast<int64_t>(block) * kQThreads + threadIdx.x;
+    const int64_t nv = qt.vec ? n / NV : 0;
     int64_t i = tid0;
     // kAmaxUnroll independent 16-byte loads in flight per lane: the grid is
-    // small (see launch_quant), so each lane must keep several loads going
+    // small (see kSlots), so each lane must keep several loads going
     constexpr int U = kAmaxUnroll;
     for (; i + (U - 1) * stride < nv; i += U * stride) {
         uint32_t w[U][4];
@@ -62,20 +105,36 @@ __global__ __launch_bounds__(kQThreads) void amax_kernel(const T* __restrict__ x
         for (int e = 0; e < NV; ++e) m = fmaxf(m, fabsf(elem<T>(w, e)));
     }
     for (int64_t i = nv * NV + tid0; i < n; i += stride) m = fmaxf(m, fabsf(ld(x, i)));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float b = part[0];
-        for (int w = 1; w < kQThreads / 64; ++w) b = fmaxf(b, part[w]);
-        atomicMax(amax_bits, __float_as_uint(b));
-    }
+    m = block_max(m);
+    if (threadIdx.x != 0) return;
+    if (a.shared_word) atomicMax(qt.maxima, __float_as_uint(m));
+    else qt.maxima[block] = __float_as_uint(m);
 }
 
-__device__ __forceinline__ float quant_scale(const uint32_t* amax_bits) {
-    const float amax = __uint_as_float(amax_bits[0]);
-    return fmaxf(amax / 448.f, 1e-12f);
-}
+// x / scale, clamped, as the correctly rounded quotient would be coded.  A
+// true fp32 division is about ten operations per element, which the pass
+// waited for.  For 16-bit x the quotient from the scale's reciprocal and one
+// residual step (Markstein, 1990) takes three, and its codes equal the true
+// division's for every pair of a 16-bit x and a 16-bit amax >= |x|; copysign
+// keeps the sign of a zero, and an infinite scale takes no residual (finite x
+// give zeros, infinite ones NaN, as the division does).  fp32 x divide.
+template <typename T>
+struct Quotient {
+    float scale, inv;
+    __device__ __forceinline__ explicit Quotient(float s) : scale(s), inv(1.f / s) {
+        if constexpr (sizeof(T) == 2) scale = s == __builtin_inff() ? 0.f : s;
+    }
+    __device__ __forceinline__ float operator()(float x) const {
+        float v;
+        if constexpr (sizeof(T) == 2) {
+            const float q = x * inv;
+            v = copysignf(fmaf(fmaf(-q, scale, x), inv, q), x);
+        } else {
+            v = x / scale;
+        }
+        return fminf(fmaxf(v, -448.f), 448.f);
+    }
+};
 
 // Round-to-nearest-even conversion of a value already clamped to +-448.
 __device__ __forceinline__ uint32_t to_e4m3(float v) {
@@ -89,20 +148,30 @@ __device__ __forceinline__ uint32_t pack_e4m3(float v0, float v1, float v2, floa
 }
 
 template <typename T>
-__global__ __launch_bounds__(kQThreads) void quant_kernel(const T* __restrict__ x, uint8_t* __restrict__ x8, int64_t n,
-                                                          const uint32_t* amax_bits, float* scale_out, int vec) {
+__global__ __launch_bounds__(kQThreads) void quant_kernel(const QuantArgs a) {
     constexpr int NV = 16 / sizeof(T);  // elements per 16-byte load
-    const float scale = quant_scale(amax_bits);
-    if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = scale;
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kQThreads;
-    const int64_t tid0 = static_cast<int64_t>(blockIdx.x) * kQThreads + threadIdx.x;
-    if (vec) {
+    int ti = 0;
+    while (ti + 1 < a.count && blockIdx.x >= a.t[ti + 1].quant_begin) ++ti;
+    const QuantTensor& qt = a.t[ti];
+    const T* __restrict__ x = static_cast<const T*>(qt.x);
+    uint8_t* __restrict__ x8 = qt.x8;
+    const int64_t n = qt.n;
+    const unsigned block = blockIdx.x - qt.quant_begin;
+    float m = 0.f;
+    const unsigned words = a.shared_word ? 1u : qt.amax_blocks;
+    for (unsigned w = threadIdx.x; w < words; w += kQThreads) m = fmaxf(m, __uint_as_float(qt.maxima[w]));
+    const float scale = fmaxf(block_max(m) / 448.f, 1e-12f);
+    const Quotient<T> quotient(scale);
+    if (block == 0 && threadIdx.x == 0) qt.scale_out[0] = scale;
+    const int64_t stride = static_cast<int64_t>(qt.quant_blocks) * kQThreads;
+    const int64_t tid0 = static_cast<int64_t>(block) * kQThreads + threadIdx.x;
+    if (qt.vec) {
         // NV elements per thread and step: one 16-byte load, NV / 4 word stores
         const int64_t nv = n / NV;
         auto emit = [&](int64_t j, const uint32_t* w) {
             float v[NV];
 #pragma unroll
-            for (int e = 0; e < NV; ++e) v[e] = fminf(fmaxf(elem<T>(w, e) / scale, -448.f), 448.f);
+            for (int e = 0; e < NV; ++e) v[e] = quotient(elem<T>(w, e));
             if constexpr (NV == 8) {
                 *reinterpret_cast<uint2*>(x8 + j * NV) =
                     uint2{pack_e4m3(v[0], v[1], v[2], v[3]), pack_e4m3(v[4], v[5], v[6], v[7])};
@@ -123,9 +192,9 @@ __global__ __launch_bounds__(kQThreads) void quant_kernel(const T* __restrict__ 
             load_words(x + i * NV, w);
             emit(i, w);
         }
-        if (blockIdx.x == 0) {
+        if (block == 0) {
             for (int64_t i = nv * NV + threadIdx.x; i < n; i += kQThreads) {
-                const float v = fminf(fmaxf(ld(x, i) / scale, -448.f), 448.f);
+                const float v = quotient(ld(x, i));
                 x8[i] = static_cast<uint8_t>(to_e4m3(v));
             }
         }
@@ -137,34 +206,58 @@ __global__ __launch_bounds__(kQThreads) void quant_kernel(const T* __restrict__ 
         uint32_t word = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float v = fminf(fmaxf(ld(x, 4 * i + e) / scale, -448.f), 448.f);
+            const float v = quotient(ld(x, 4 * i + e));
             word |= to_e4m3(v) << (8 * e);
         }
         reinterpret_cast<uint32_t*>(x8)[i] = word;
     }
-    if (blockIdx.x == 0) {
+    if (block == 0) {
         for (int64_t i = 4 * n4 + threadIdx.x; i < n; i += kQThreads) {
-            const float v = fminf(fmaxf(ld(x, i) / scale, -448.f), 448.f);
+            const float v = quotient(ld(x, i));
             x8[i] = static_cast<uint8_t>(to_e4m3(v));
         }
     }
 }
 
+// Deals out the blocks of both passes by size and launches them.
 template <typename T>
-int launch_quant(const void* x, void* x8, int64_t n, float* amax_ws, float* scale_out, hipStream_t st) {
-    uint32_t* ab = reinterpret_cast<uint32_t*>(amax_ws);
-    fill_zero_u32<<<1, 1, 0, st>>>(ab);
-    // 16-byte steps need x 16-byte aligned and x8 aligned to the step's
-    // output (8 or 4 bytes; the entry point requires 4)
+int launch_quant(QuantArgs& a, hipStream_t st) {
     constexpr int NV = 16 / sizeof(T);
-    const int vec = aligned16(x) && (reinterpret_cast<uintptr_t>(x8) % NV) == 0 ? 1 : 0;
-    const int64_t want = (n + kQThreads * 4 * NV - 1) / (kQThreads * 4 * NV);
-    const unsigned blocks = static_cast<unsigned>(want < 1 ? 1 : (want > 4096 ? 4096 : want));
-    const unsigned ablocks = blocks > kAmaxBlocks ? kAmaxBlocks : blocks;
-    amax_kernel<T><<<ablocks, kQThreads, 0, st>>>(static_cast<const T*>(x), n, ab, vec);
-    quant_kernel<T><<<blocks, kQThreads, 0, st>>>(static_cast<const T*>(x), static_cast<uint8_t*>(x8), n, ab,
-                                                  scale_out, vec);
+    constexpr int64_t kPerBlock = kQThreads * 4 * NV;
+    double total = 0;
+    for (int i = 0; i < a.count; ++i) total += static_cast<double>(a.t[i].n);
+    const unsigned amax_limit = a.shared_word ? kAmaxAtomicBlocks : kSlots;
+    unsigned amax_grid = 0, quant_grid = 0;
+    for (int i = 0; i < a.count; ++i) {
+        QuantTensor& t = a.t[i];
+        // 16-byte steps need x 16-byte aligned and x8 aligned to the step's
+        // output (8 or 4 bytes; the entry points require 4)
+        t.vec = aligned16(t.x) && (reinterpret_cast<uintptr_t>(t.x8) % NV) == 0 ? 1 : 0;
+        const int64_t want = (t.n + kPerBlock - 1) / kPerBlock;
+        const double share = total > 0 ? static_cast<double>(t.n) / total : 0;
+        auto blocks = [&](unsigned limit) {
+            const int64_t most = static_cast<int64_t>(share * limit);
+            const int64_t b = want < most ? want : most;
+            return static_cast<unsigned>(b < 1 ? 1 : b);
+        };
+        t.amax_begin = amax_grid;
+        t.quant_begin = quant_grid;
+        amax_grid += t.amax_blocks = blocks(amax_limit);
+        quant_grid += t.quant_blocks = blocks(kQuantBlocks);
+    }
+    amax_kernel<T><<<amax_grid, kQThreads, 0, st>>>(a);
+    quant_kernel<T><<<quant_grid, kQThreads, 0, st>>>(a);
     return status_from_launch();
+}
+
+int launch_quant(QuantArgs& a, int dtype, hipStream_t st) {
+    if (dtype != SA_F32 && dtype != SA_F16 && dtype != SA_BF16) return SA_ERR_BAD_DTYPE;
+    if (a.shared_word) fill_zero_u32<<<1, 1, 0, st>>>(a.t[0].maxima);
+    switch (dtype) {
+        case SA_F32: return launch_quant<float>(a, st);
+        case SA_F16: return launch_quant<f16>(a, st);
+        default: return launch_quant<bf16>(a, st);
+    }
 }
 
 }  // namespace
@@ -176,11 +269,33 @@ extern "C" int sa_fp8_quantize(const void* x, void* x8, int64_t n, int dtype, fl
     if (n < 0) return SA_ERR_BAD_SHAPE;
     if (!amax_ws || !scale_out || (n > 0 && (!x || !x8))) return SA_ERR_NULL_POINTER;
     if ((reinterpret_cast<uintptr_t>(x8) & 3u) != 0) return SA_ERR_BAD_STRIDE;
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    switch (dtype) {
-        case SA_F32: return launch_quant<float>(x, x8, n, amax_ws, scale_out, st);
-        case SA_F16: return launch_quant<f16>(x, x8, n, amax_ws, scale_out, st);
-        case SA_BF16: return launch_quant<bf16>(x, x8, n, amax_ws, scale_out, st);
-        default: return SA_ERR_BAD_DTYPE;
+    QuantArgs a{};
+    a.count = 1;
+    a.shared_word = 1;
+    a.t[0].x = x;
+    a.t[0].x8 = static_cast<uint8_t*>(x8);
+    a.t[0].n = n;
+    a.t[0].maxima = reinterpret_cast<uint32_t*>(amax_ws);
+    a.t[0].scale_out = scale_out;
+    return launch_quant(a, dtype, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int sa_fp8_quantize_many(int count, const void* const* x, void* const* x8, const int64_t* n, int dtype,
+                                    float* amax_ws, float* scales_out, sa_stream_t stream) {
+    using namespace sa;
+    if (count < 1 || count > kMaxTensors) return SA_ERR_BAD_SHAPE;
+    if (!x || !x8 || !n || !amax_ws || !scales_out) return SA_ERR_NULL_POINTER;
+    QuantArgs a{};
+    a.count = count;
+    for (int i = 0; i < count; ++i) {
+        if (n[i] < 0) return SA_ERR_BAD_SHAPE;
+        if (n[i] > 0 && (!x[i] || !x8[i])) return SA_ERR_NULL_POINTER;
+        if ((reinterpret_cast<uintptr_t>(x8[i]) & 3u) != 0) return SA_ERR_BAD_STRIDE;
+        a.t[i].x = x[i];
+        a.t[i].x8 = static_cast<uint8_t*>(x8[i]);
+        a.t[i].n = n[i];
+        a.t[i].maxima = reinterpret_cast<uint32_t*>(amax_ws) + static_cast<int64_t>(i) * kSlots;
+        a.t[i].scale_out = scales_out + i;
     }
+    return launch_quant(a, dtype, reinterpret_cast<hipStream_t>(stream));
 }

@@ -17,6 +17,7 @@ LIB_PATH = Path(os.environ.get("SMOOTH_ATTN_LIB") or Path(__file__).resolve().pa
 
 # Element-type codes (SA_F32 ... in the header).
 SA_F32, SA_F16, SA_BF16, SA_FP8_E4M3FN = 0, 1, 2, 3
+SA_FP8_AMAX_WORDS = 1024
 
 
 def paged_dtypes(q_type: int, cache_type: int) -> int:
@@ -65,6 +66,8 @@ SIGNATURES = {
                                 _I64P, _I64P, _I64P, _I64P, _I64P, c_float, c_int, c_int, c_int, c_void_p, c_int64,
                                 c_void_p]),
     "sa_fp8_quantize": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p]),
+    "sa_fp8_quantize_many": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), _I64P, c_int,
+                                     c_void_p, c_void_p, c_void_p]),
     "sa_flash_fp8_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_int, c_int, c_int, c_int, c_int, _I64P, _I64P, _I64P, _I64P,
                                  c_float, c_int, c_int, c_void_p]),

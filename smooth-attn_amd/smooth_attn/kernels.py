@@ -863,18 +863,29 @@ FP8_MAX = 448.0
 
 def _quantize_to_fp8_device(x):
     """(x8, scale) with the scale left on the device (no host sync)."""
+    return _quantize_many_to_fp8_device(x)[0]
+
+
+def _quantize_many_to_fp8_device(*xs):
+    """[(x8, scale)] of one to four tensors of one dtype on one device, each
+    with its own scale, in the two launches that one tensor takes."""
+    x = xs[0]
     _check_same_device("x", x)
     if x.dtype not in _DTYPE_CODE:
         raise ValueError(f"cannot quantise dtype {x.dtype}")
-    xc = x.detach().contiguous()
-    x8 = torch.empty(xc.shape, dtype=torch.float8_e4m3fn, device=x.device)
-    ws = torch.empty(2, dtype=torch.float32, device=x.device)
+    count = len(xs)
+    xc = [t.detach().contiguous() for t in xs]
+    x8 = [torch.empty(t.shape, dtype=torch.float8_e4m3fn, device=x.device) for t in xc]
+    scales = torch.empty(count, dtype=torch.float32, device=x.device)
+    ws = torch.empty(count * _lib.SA_FP8_AMAX_WORDS, dtype=torch.float32, device=x.device)
+    ptrs = ctypes.c_void_p * count
     lib = _lib.load()
     with _device_of(x):
-        st = lib.sa_fp8_quantize(xc.data_ptr(), x8.data_ptr(), xc.numel(), _DTYPE_CODE[xc.dtype],
-                                 ws.data_ptr(), ws.data_ptr() + 4, _stream(xc))
-    _lib.check(st, "sa_fp8_quantize")
-    return x8, ws[1]
+        st = lib.sa_fp8_quantize_many(count, ptrs(*[t.data_ptr() for t in xc]), ptrs(*[t.data_ptr() for t in x8]),
+                                      (ctypes.c_int64 * count)(*[t.numel() for t in xc]), _DTYPE_CODE[x.dtype],
+                                      ws.data_ptr(), scales.data_ptr(), _stream(x))
+    _lib.check(st, "sa_fp8_quantize_many")
+    return list(zip(x8, scales.unbind()))
 
 
 def _quantize_to_fp8(x):
@@ -970,12 +981,13 @@ def sp2norm_fp8_flash_attention(q, k, v, *, scale=None, window_size=0, quantize_
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     n_kv_groups = H_q // H_kv
-    q8, q_s = _quantize_to_fp8_device(q)
-    k8, k_s = _quantize_to_fp8_device(k)
-    if quantize_v:
-        v8, v_s = _quantize_to_fp8_device(v)
+    xs = (q, k, v) if quantize_v else (q, k)
+    if all(x.dtype == q.dtype for x in xs):
+        codes = _quantize_many_to_fp8_device(*xs)
     else:
-        v8, v_s = v.detach().to(torch.bfloat16), None
+        codes = [_quantize_to_fp8_device(x) for x in xs]
+    (q8, q_s), (k8, k_s) = codes[:2]
+    v8, v_s = codes[2] if quantize_v else (v.detach().to(torch.bfloat16), None)
     o, _row_sums = _sp2norm_fp8_flash_fwd(q8, k8, v8, q_s, k_s, v_s, scale, n_kv_groups, window_size)
     return o
 
