@@ -435,6 +435,22 @@ int sa_paged_kv_append(const void* k_new, const void* v_new, void* k_cache,
                        const int64_t* vc_strides, int64_t bt_stride, int dtype,
                        sa_stream_t stream);
 
+/*
+ * The same, and in the same launch lens_out[i] = context_lens[i] + n_new for
+ * i < lens_count (>= 0; context_lens holds at least B and lens_count entries;
+ * lens_out does not overlap context_lens).
+ */
+int sa_paged_kv_append_lens(const void* k_new, const void* v_new,
+                            void* k_cache, void* v_cache,
+                            const int32_t* block_table,
+                            const int32_t* context_lens, int32_t* lens_out,
+                            int64_t lens_count, int B, int Hkv, int n_new,
+                            int D, int page_size, int max_pages, int n_pages,
+                            const int64_t* new_strides,
+                            const int64_t* kc_strides,
+                            const int64_t* vc_strides, int64_t bt_stride,
+                            int dtype, sa_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -54,7 +54,7 @@ struct Abi {
     decltype(&sa_flash_bwd_workspace_size) flash_bwd_workspace_size = nullptr;
     decltype(&sa_paged_decode) paged_decode = nullptr;
     decltype(&sa_paged_decode_workspace_size) paged_decode_workspace_size = nullptr;
-    decltype(&sa_paged_kv_append) paged_kv_append = nullptr;
+    decltype(&sa_paged_kv_append_lens) paged_kv_append_lens = nullptr;
 } abi;
 
 template <typename F>
@@ -80,7 +80,7 @@ PyObject* py_bind(PyObject*, PyObject* table) {
         !bind_one(table, "sa_flash_bwd_workspace_size", abi.flash_bwd_workspace_size) ||
         !bind_one(table, "sa_paged_decode", abi.paged_decode) ||
         !bind_one(table, "sa_paged_decode_workspace_size", abi.paged_decode_workspace_size) ||
-        !bind_one(table, "sa_paged_kv_append", abi.paged_kv_append))
+        !bind_one(table, "sa_paged_kv_append_lens", abi.paged_kv_append_lens))
         return nullptr;
     Py_RETURN_NONE;
 }
@@ -423,16 +423,16 @@ PyObject* py_paged_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!paging_ok(*k, B, Hkv, D, block_size, *k, *v, *table, *lens) || D % (16 / k->element_size()) != 0 ||
         !operand_ok(*kn) || !operand_ok(*vn) || kn->strides() != vn->strides() || B > INT32_MAX || n_new > INT32_MAX)
         Py_RETURN_NONE;
-    {
-        const c10::DeviceGuard guard(k->device());
-        check(abi.paged_kv_append(kn->data_ptr(), vn->data_ptr(), k->data_ptr(), v->data_ptr(),
-                                  table->data_ptr<int32_t>(), lens->data_ptr<int32_t>(), static_cast<int>(B),
-                                  static_cast<int>(Hkv), static_cast<int>(n_new), static_cast<int>(D), block_size,
-                                  static_cast<int>(table->size(1)), static_cast<int>(k->size(0)), strides(*kn),
-                                  strides(*k), strides(*v), table->stride(0), code, stream_of(*k)),
-              "sa_paged_kv_append");
-    }
-    return THPVariable_Wrap(at::add(*lens, static_cast<int64_t>(n_new)));
+    const c10::DeviceGuard guard(k->device());
+    Tensor out = at::empty(lens->sizes(), lens->options());
+    check(abi.paged_kv_append_lens(kn->data_ptr(), vn->data_ptr(), k->data_ptr(), v->data_ptr(),
+                                   table->data_ptr<int32_t>(), lens->data_ptr<int32_t>(), out.data_ptr<int32_t>(),
+                                   lens->numel(), static_cast<int>(B), static_cast<int>(Hkv),
+                                   static_cast<int>(n_new), static_cast<int>(D), block_size,
+                                   static_cast<int>(table->size(1)), static_cast<int>(k->size(0)), strides(*kn),
+                                   strides(*k), strides(*v), table->stride(0), code, stream_of(*k)),
+          "sa_paged_kv_append_lens");
+    return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
 
