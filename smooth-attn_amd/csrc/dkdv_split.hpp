@@ -1,6 +1,6 @@
-// Host-side pieces of the dK/dV query-range split shared by the backward
-// kernels for head dims up to 128 and for head dims 136..512: the makespan
-// estimate the split count is chosen by, and a small cache of chosen counts.
+// Host-side pieces of the dK/dV query-range split: the makespan estimate by
+// which the backward for head dims 136..512 chooses its split count, and a
+// small cache of choices shared with the backward for head dims up to 128.
 #pragma once
 
 #include <algorithm>
