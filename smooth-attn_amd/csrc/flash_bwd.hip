@@ -80,6 +80,7 @@ struct BwdParams {
     // (summed by bwd_split_reduce_kernel); 1 = no split, results stored directly
     int n_split;
     float* part;
+    int dq_units, kv_units;    // units_per_group of the two grids
     int dq_groups, kv_groups;  // row groups per block of the two kernels (1 or 2, see merge_groups)
 };
 
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? 2 : 1) void flash_bwd_d
 
     const int nqb = (p.T + kBwdBQ - 1) / kBwdBQ;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, kBwdXcdSlots, true, step, unit, sub);
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, p.dq_units, step, unit, sub);
     const int qb = nqb - 1 - step;  // heaviest (latest) query blocks first
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? kBwdDkdvMinBlocks : 1) 
     }
     int kb, unit, sub;
     // earliest key blocks see the most queries: first
-    grouped_block(ob, p.B * p.Hkv, 1, nkb, kBwdXcdSlots, true, kb, unit, sub);
+    grouped_block(ob, p.B * p.Hkv, 1, nkb, p.kv_units, kb, unit, sub);
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
     const int T_ = p.T;
@@ -1069,6 +1070,9 @@ extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, cons
     const BwdPlan plan = choose_bwd_plan(B, Hkv, T, prm.G, window_size, D, max_split, !exact_math);
     prm.n_split = plan.n_split;
     prm.part = plan.n_split > 1 ? static_cast<float*>(workspace) : nullptr;
+    // the block order's group sizes, worked out here rather than before every block's first load
+    prm.dq_units = units_per_group(B * Hkv, prm.G, (T + kBwdBQ - 1) / kBwdBQ, kBwdXcdSlots, true);
+    prm.kv_units = units_per_group(B * Hkv, 1, (T + kBwdBK - 1) / kBwdBK, kBwdXcdSlots, true);
     prm.dq_groups = plan.dq_groups;
     prm.kv_groups = plan.kv_groups;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -95,15 +95,25 @@ __device__ __forceinline__ V lds_read_tr16_pair(const void* p0, const void* p1) 
 // -> 934 / 3080), and so do equal steps ([2,32/8,3000] window 1024 forward 122
 // -> 125).
 constexpr int kOneGroupRounds = 8;
-__device__ __forceinline__ void grouped_block(int id, int n_units, int n_sub, int n_steps, int xcd_slots,
-                                              bool uneven, int& step, int& unit, int& sub) {
+__host__ __device__ __forceinline__ int units_per_group(int n_units, int n_sub, int n_steps, int xcd_slots,
+                                                        bool uneven) {
+    // blocks of a unit (none in an empty call, which launches nothing), units of an XCD
+    const int per = n_sub * n_steps > 0 ? n_sub * n_steps : 1, units = n_units >> 3;
+    int gu = (xcd_slots + per - 1) / per;
+    if (gu < 1) gu = 1;
+    if (gu > units) gu = units;
+    if (uneven && units * per <= kOneGroupRounds * xcd_slots && gu * per % xcd_slots != 0) gu = units;
+    return gu;
+}
+
+// gu: units_per_group of the same grid (read only where n_units is a multiple
+// of 8, and then at least 1).
+__device__ __forceinline__ void grouped_block(int id, int n_units, int n_sub, int n_steps, int gu, int& step,
+                                              int& unit, int& sub) {
     if ((n_units & 7) == 0) {
         const int x = id & 7;
         const int j = id >> 3;
         const int nh = (n_units >> 3) * n_sub;  // (unit, sub) pairs on this XCD
-        int gu = min(max(1, (xcd_slots + n_sub * n_steps - 1) / (n_sub * n_steps)), n_units >> 3);
-        if (uneven && nh * n_steps <= kOneGroupRounds * xcd_slots && gu * n_sub * n_steps % xcd_slots != 0)
-            gu = n_units >> 3;
         const int gh = gu * n_sub;  // pairs per group
         const int grp = j / (gh * n_steps);
         const int r = j - grp * (gh * n_steps);

@@ -242,7 +242,7 @@ int fill_params(FlashParams& prm, const void* q, const void* k, const void* v, v
     prm.T = T;
     prm.G = Hq / Hkv;
     prm.window = window_size;
-    prm.nqb = (T + Split<1>::BQ - 1) / Split<1>::BQ;
+    set_grid(prm, Split<1>::BQ);
     prm.dr = D;
     prm.scale = scale;
     return 0;

@@ -65,7 +65,8 @@ struct FlashParams {
     const float* rope_cos;  // RoPE tables [T, D/2] fp32 (RoPE variant only)
     const float* rope_sin;
     int64_t qs[4], ks[4], vs[4], os[4];
-    int B, Hq, Hkv, T, G, window, nqb;
+    int B, Hq, Hkv, T, G, window;
+    int nqb, group_units;  // query blocks, and units_per_group of the grid (set_grid)
     int dr;  // head dim of the tensors (<= D, a multiple of 8; columns past it read as zero, are not stored)
     float scale;
 };
@@ -145,13 +146,23 @@ __device__ __forceinline__ u32x4 tile_load16(const T* p) {
 // (units) and the query heads sharing each (sub), heaviest query block first;
 // one block per CU, so an XCD runs 32 at once.
 constexpr int kBlocksPerXcd = 32;
-__device__ __forceinline__ void block_coords(const FlashParams& p, int& qb, int& b, int& hq) {
-    int step, unit, sub;
+
+// Query blocks of bq rows and their order.  The group size is worked out here,
+// once: in the kernel its divisions stood before every block's first load
+// (forward, means of two runs: [2,32/8,1152,96] 35.8 -> 35.3 us,
+// [1,32/8,512,128] 11.6 -> 11.4, [8,32,878,80] 86.3 -> 85.9).
+inline void set_grid(FlashParams& p, int bq) {
+    p.nqb = (p.T + bq - 1) / bq;
     // (under a window of up to half the rows most query blocks walk equally
     // many tiles; and groups of one KV head that fill the XCD by themselves
     // are balanced within 5%, where the L2 hits count more)
     const bool uneven = (p.window <= 0 || 2 * p.window > p.T) && p.G * p.nqb <= kBlocksPerXcd;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, p.nqb, kBlocksPerXcd, uneven, step, unit, sub);
+    p.group_units = units_per_group(p.B * p.Hkv, p.G, p.nqb, kBlocksPerXcd, uneven);
+}
+
+__device__ __forceinline__ void block_coords(const FlashParams& p, int& qb, int& b, int& hq) {
+    int step, unit, sub;
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, p.nqb, p.group_units, step, unit, sub);
     qb = p.nqb - 1 - step;
     b = unit / p.Hkv;
     hq = (unit - b * p.Hkv) * p.G + sub;
@@ -763,7 +774,7 @@ bool fold_scale_ok(float scale) {
 // One launch of the kernel with key split KS (not for exact math).
 template <typename T, int D, bool QK8, bool V8, bool ROPE, int KS>
 int launch_flash_split(FlashParams prm, hipStream_t st) {
-    prm.nqb = (prm.T + Split<KS>::BQ - 1) / Split<KS>::BQ;
+    set_grid(prm, Split<KS>::BQ);
     const dim3 grid(static_cast<unsigned>(prm.nqb) * prm.B * prm.Hq);
     if constexpr (kCanFold<T, QK8, D>) {
         if (fold_scale_ok<QK8>(prm.scale)) {

@@ -212,7 +212,8 @@ __global__ __launch_bounds__(64 * WideCfg<D>::NW) void flash_fwd_wide_kernel(Wid
     const int T_ = p.T;
     const int nqb = (T_ + kFRows - 1) / kFRows;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, 32, true, step, unit, sub);  // heaviest query blocks first
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, units_per_group(p.B * p.Hkv, p.G, nqb, 32, true), step, unit,
+                  sub);  // heaviest query blocks first
     const int qb = nqb - 1 - step;
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
@@ -432,7 +433,8 @@ __global__ __launch_bounds__(64 * WideCfg<D>::NW) void flash_bwd_dq_wide_kernel(
     const int T_ = p.T;
     const int nqb = (T_ + kFRows - 1) / kFRows;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, 32, false, step, unit, sub);
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, units_per_group(p.B * p.Hkv, p.G, nqb, 32, false), step, unit,
+                  sub);
     const int qb = nqb - 1 - step;
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
