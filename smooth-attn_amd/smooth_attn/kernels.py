@@ -107,11 +107,24 @@ def _resolve_family(alpha, theta, power, family):
     return family
 
 
+class _NothingOrdinary:
+    """The native call path's answers where no tensor can be on a GPU."""
+
+    @staticmethod
+    def _none(*_):
+        return None
+
+    norm_out = causal_norm = flash = paged = paged_append = _none
+
+
 def _native():
     """The native call path (csrc/host/host.cpp).  It takes the calls whose
     tensors the kernels can use as they are and answers None (or False) to
-    every other one, which then goes through the Python path below it; on a
-    machine without a GPU nothing is ordinary, and the Python path raises."""
+    every other one, which then goes through the Python path below it.  Until
+    CUDA is initialised no tensor is on a GPU and no call is ordinary: the
+    libraries are not loaded for it, and the Python path's checks refuse it."""
+    if _lib._host is None and not torch.cuda.is_initialized():
+        return _NothingOrdinary
     return _lib.host()
 
 
