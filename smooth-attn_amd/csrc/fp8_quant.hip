@@ -10,7 +10,7 @@
 // HBM binds the large sizes and the launches the small ones: q, k and v of a
 // [2,32/8,8192,128] forward 107 -> 86 us (31.5 us at 6.4 TB/s, then 54 us at
 // 5.6 TB/s), its whole call 945 -> 922 us; a [1,32/8,2048,128] call
-// 83 -> 63 us.  Walking the second pass backwards, towards what the first
+// 83 -> 63 us, then 55 (load_words_cached).  Walking the second pass backwards, towards what the first
 // read last, changed nothing.  Both passes
 // read 16 bytes per lane and load when x is 16-byte aligned (the remainder,
 // and unaligned inputs, element by element), several loads in flight per lane.
@@ -50,6 +50,21 @@ struct QuantArgs {
 };
 
 __global__ void fill_zero_u32(uint32_t* p) { p[0] = 0u; }
+
+// 16-byte loads that leave their lines in the caches: the second pass reads
+// what the first one has just read, from the caches for calls up to their
+// size.  Nontemporal loads -> these, whole calls (bf16 inputs):
+// [1,32/8,2048,128] 61.1 -> 55.3 us, [8,32/8,1024,128] 124.7 -> 120.5,
+// [4,16/2,3001,64] 115.4 -> 110.8, [1,32/8,8192,128] 467.9 -> 463.7,
+// [2,32/8,8192,128] (201 MB of inputs) unchanged.
+template <typename T>
+__device__ __forceinline__ void load_words_cached(const T* p, uint32_t* words) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+    words[0] = v.x;
+    words[1] = v.y;
+    words[2] = v.z;
+    words[3] = v.w;
+}
 
 template <typename T>
 __device__ __forceinline__ float ld(const T* p, int64_t i) { return to_f32(p[i]); }
@@ -92,7 +107,7 @@ __global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
     for (; i + (U - 1) * stride < nv; i += U * stride) {
         uint32_t w[U][4];
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_words(x + (i + u * stride) * NV, w[u]);
+        for (int u = 0; u < U; ++u) load_words_cached(x + (i + u * stride) * NV, w[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -100,7 +115,7 @@ __global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
     }
     for (; i < nv; i += stride) {
         uint32_t w[4];
-        load_words(x + i * NV, w);
+        load_words_cached(x + i * NV, w);
 #pragma unroll
         for (int e = 0; e < NV; ++e) m = fmaxf(m, fabsf(elem<T>(w, e)));
     }
@@ -182,14 +197,14 @@ __global__ __launch_bounds__(kQThreads) void quant_kernel(const QuantArgs a) {
         int64_t i = tid0;
         for (; i + stride < nv; i += 2 * stride) {  // two loads in flight per lane
             uint32_t w0[4], w1[4];
-            load_words(x + i * NV, w0);
-            load_words(x + (i + stride) * NV, w1);
+            load_words_cached(x + i * NV, w0);
+            load_words_cached(x + (i + stride) * NV, w1);
             emit(i, w0);
             emit(i + stride, w1);
         }
         for (; i < nv; i += stride) {
             uint32_t w[4];
-            load_words(x + i * NV, w);
+            load_words_cached(x + i * NV, w);
             emit(i, w);
         }
         if (block == 0) {
