@@ -216,21 +216,27 @@ struct CausalNorm : public torch::autograd::Function<CausalNorm> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         if (!ctx->needs_input_grad(0)) return {Tensor(), Tensor(), Tensor(), Tensor()};
-        const Tensor x = ctx->get_saved_variables()[0];
+        const Tensor saved = ctx->get_saved_variables()[0];
         Tensor g = grads[0];
-        TORCH_CHECK_VALUE(g.is_cuda() && g.device() == x.device(), "grad_output must live on the same CUDA device as x");
+        TORCH_CHECK_VALUE(g.is_cuda() && g.device() == saved.device(),
+                          "grad_output must live on the same CUDA device as x");
+        TORCH_CHECK_VALUE(float_code(code_of(saved.scalar_type())) && saved.sizes() == g.sizes(),
+                          "the saved x must have grad_output's shape and a dtype of the fused kernels");
+        const int64_t cols = saved.size(-1);
+        // (unpack hooks may hand back another layout or type than forward saved)
+        Tensor x = saved.reshape({-1, cols});
+        if (x.stride(1) != 1 || x.stride(0) < cols) x = x.contiguous();
         if (g.scalar_type() != at::kFloat && g.scalar_type() != x.scalar_type()) g = g.to(at::kFloat);
         g = g.contiguous();
         Tensor dx = at::empty_like(x);
-        const int64_t cols = x.size(-1);
         const c10::DeviceGuard guard(x.device());
-        check(abi.norm_bwd(x.data_ptr(), g.data_ptr(), dx.data_ptr(), x.numel() / cols, cols, cols, cols, cols,
+        check(abi.norm_bwd(x.data_ptr(), g.data_ptr(), dx.data_ptr(), x.size(0), cols, x.stride(0), cols, dx.stride(0),
                            code_of(x.scalar_type()), code_of(g.scalar_type()), 1,
                            static_cast<float>(ctx->saved_data["alpha"].toDouble()),
                            static_cast<float>(ctx->saved_data["theta"].toDouble()),
                            static_cast<int>(ctx->saved_data["power"].toInt()), stream_of(x)),
               "sa_norm_bwd");
-        return {dx, Tensor(), Tensor(), Tensor()};
+        return {dx.view(saved.sizes()), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -287,6 +293,26 @@ void flash_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const FlashCal
           "sa_flash_fwd");
 }
 
+// What backward reads: q, k, v, o and the row sums as forward saved them, or
+// as unpack hooks hand them back.
+void check_saved(const variable_list& saved, const Tensor& grad) {
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &row_sums = saved[4];
+    for (const Tensor* t : {&q, &k, &v, &o, &row_sums, &grad})
+        TORCH_CHECK_VALUE(t->is_cuda() && t->device() == q.device(),
+                          "attention tensors must live on the same CUDA device as q");
+    TORCH_CHECK_VALUE(float_code(code_of(q.scalar_type())) && k.scalar_type() == q.scalar_type() &&
+                          v.scalar_type() == q.scalar_type(),
+                      "fused attention expects bf16, fp16 or fp32 q/k/v of one dtype, got ", q.scalar_type(), "/",
+                      k.scalar_type(), "/", v.scalar_type());
+    TORCH_CHECK_VALUE(o.scalar_type() == q.scalar_type() && row_sums.scalar_type() == at::kFloat,
+                      "the saved output must have q's dtype and the saved row sums fp32");
+    TORCH_CHECK_VALUE(q.sizes() == grad.sizes() && o.sizes() == grad.sizes() && k.dim() == 4 && v.sizes() == k.sizes() &&
+                          k.size(0) == q.size(0) && k.size(1) > 0 && q.size(1) % k.size(1) == 0 &&
+                          k.size(2) == q.size(2) && k.size(3) == q.size(3) &&
+                          row_sums.sizes() == q.sizes().slice(0, 3),
+                      "the saved attention tensors must have the shapes that forward saved");
+}
+
 struct Flash : public torch::autograd::Function<Flash> {
     static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, double scale,
                           int64_t window, bool exact) {
@@ -300,14 +326,17 @@ struct Flash : public torch::autograd::Function<Flash> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
-        // (unpack hooks may hand back tensors of another layout)
-        const auto fix = [](const Tensor& t) { return operand_ok(t) ? t : t.clone(at::MemoryFormat::Contiguous); };
+        check_saved(saved, grads[0]);
+        // (unpack hooks may hand back tensors of another layout, or of a type that takes fewer head dims)
+        const int64_t D0 = saved[0].size(3), step = saved[0].scalar_type() == at::kFloat ? 4 : 8;
+        const int64_t pad = (step - D0 % step) % step;
+        const auto fix = [pad](const Tensor& t) {
+            if (pad != 0) return at::constant_pad_nd(t, {0, pad});
+            return operand_ok(t) ? t : t.clone(at::MemoryFormat::Contiguous);
+        };
         const Tensor q = fix(saved[0]), k = fix(saved[1]), v = fix(saved[2]), o = fix(saved[3]);
         const Tensor row_sums = saved[4].contiguous();
         const Tensor g = fix(grads[0].to(q.scalar_type()));
-        for (const Tensor* t : {&k, &v, &o, &row_sums, &g})
-            TORCH_CHECK_VALUE(t->is_cuda() && t->device() == q.device(),
-                              "attention tensors must live on the same CUDA device as q");
         const double scale = ctx->saved_data["scale"].toDouble();
         const int window = static_cast<int>(ctx->saved_data["window"].toInt());
         const bool exact = ctx->saved_data["exact"].toBool();
@@ -327,6 +356,8 @@ struct Flash : public torch::autograd::Function<Flash> {
                                static_cast<float>(scale), window, exact, code,
                                ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)),
               "sa_flash_bwd_ws");
+        for (Tensor* t : {&dq, &dk, &dv})
+            if (pad != 0) *t = t->narrow(3, 0, D0).contiguous();
         return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
     }
 };

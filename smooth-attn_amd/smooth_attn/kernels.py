@@ -373,6 +373,8 @@ def _softplus_norm_causal_backward(x, grad_output, family):
     _check_same_device("x", x, grad_output=grad_output)
     seq_len = x.shape[-1]
     x2d = x.reshape(-1, seq_len)
+    if x2d.stride(1) != 1 or x2d.stride(0) < seq_len:  # (saved-tensor hooks may hand back any layout)
+        x2d = x2d.contiguous()
     g = grad_output
     if g.dtype not in (torch.float32, x.dtype):
         g = g.float()
@@ -661,6 +663,13 @@ def _sp2norm_flash_bwd(q, k, v, o, do, row_sums, scale, n_kv_groups=1, window_si
     B, H_q, T, D = q.shape
     H_kv = k.shape[1]
     _check_flash_dtypes(q, k, v)
+    # (the kernels read these by q's type and sizes; saved-tensor hooks may have changed them)
+    if o.dtype != q.dtype or row_sums.dtype != torch.float32:
+        raise ValueError(f"the saved output must have q's dtype {q.dtype} and the saved row sums fp32, got "
+                         f"{o.dtype} and {row_sums.dtype}")
+    if (o.shape != q.shape or do.shape != q.shape or k.shape != (B, H_kv, T, D) or v.shape != k.shape
+            or row_sums.shape != (B, H_q, T)):
+        raise ValueError("the saved attention tensors must have the shapes that forward saved")
     Dk = _kernel_head_dim(D, q.dtype)
     if Dk != D:
         pad = [_pad_head_dim(t, Dk) for t in (q, k, v, o, do.to(q.dtype))]

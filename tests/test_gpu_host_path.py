@@ -253,6 +253,99 @@ def test_saved_tensor_hooks_and_checkpoint(monkeypatch):
     assert isinstance(p, RuntimeError) and isinstance(n, RuntimeError)
 
 
+def _hooked(fn, unpack, *inputs):
+    """Gradients of fn(*inputs) whose saved tensors came back through unpack."""
+    a = [t.clone(memory_format=torch.preserve_format).requires_grad_(True) for t in inputs]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), unpack):
+        y = fn(*a)
+    return torch.autograd.grad(y, a, randn(*y.shape, dtype=y.dtype, seed=9))
+
+
+def _permuted(t):  # values as before, the last two dims swapped in memory
+    return t.transpose(-1, -2).contiguous().transpose(-1, -2)
+
+
+def _padded_rows(t):  # values as before, rows 3 elements apart
+    return torch.cat([t, t[..., :3]], -1)[..., : t.shape[-1]]
+
+
+def _off_by_one(t):
+    return torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("unpack", [_permuted, _padded_rows, _off_by_one, lambda t: t.float(),
+                                    lambda t: t.to(torch.float16)])
+@pytest.mark.parametrize("shape", [(2, 3, 40, 40), (96, 96)])
+def test_norm_backward_of_unpacked_forms(monkeypatch, unpack, shape):
+    # a saved x of any layout or type of the kernels: the gradient of its values
+    x = randn(*shape)
+    p, n, took = both(monkeypatch, lambda: _hooked(smooth_attn.softplus_norm_causal, unpack, x))
+    same(p, n)
+    assert took == 1 and not isinstance(n, Exception)
+    if unpack in (_permuted, _padded_rows, _off_by_one):
+        # rows at another alignment sum in another order: fp32 noise, then at most one bf16 step
+        (want,) = _hooked(smooth_attn.softplus_norm_causal, lambda t: t, x)
+        assert torch.allclose(n[0].float(), want.float(), rtol=2.0 ** -7, atol=1e-5 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("shape", [(3, 40, 40), (40, 40)])
+def test_norm_backward_of_expanded_x(monkeypatch, shape):
+    row = randn(1, 40)
+    x = row.expand(shape).contiguous()
+    p, n, _ = both(monkeypatch, lambda: _hooked(smooth_attn.softplus_norm_causal, lambda t: row.expand(shape), x))
+    same(p, n)
+    same(n, _hooked(smooth_attn.softplus_norm_causal, lambda t: t, x))
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 40), (torch.float32, 20)])
+@pytest.mark.parametrize("unpack", [_permuted, _padded_rows, _off_by_one, lambda t: t.float()])
+def test_attention_backward_of_unpacked_forms(monkeypatch, unpack, dtype, D):
+    f = lambda q, k: smooth_attn.sp2norm_flash_attention(q, k, k, window_size=30)
+    q, k = randn(2, 4, 70, D, dtype=dtype), randn(2, 2, 70, D, dtype=dtype, seed=1)
+    fix = lambda t: unpack(t) if t.dim() == 4 else t  # (the row sums stay fp32 and dense)
+    p, n, took = both(monkeypatch, lambda: _hooked(f, fix, q, k))
+    same(p, n)
+    assert took == 1 and not isinstance(n, Exception)
+    if unpack in (_permuted, _padded_rows, _off_by_one):
+        for a, b in zip(n, _hooked(f, lambda t: t, q, k)):
+            assert torch.equal(a, b)
+
+
+def test_attention_backward_of_a_type_with_fewer_head_dims(monkeypatch):
+    # fp32 takes D = 20, the 16-bit types multiples of 8: padded, as the Python path does
+    f = lambda q, k: smooth_attn.sp2norm_flash_attention(q, k, k)
+    half = lambda t: t.to(torch.bfloat16) if t.dim() == 4 else t
+    p, n, _ = both(monkeypatch, lambda: _hooked(f, half, randn(1, 4, 33, 20, dtype=torch.float32),
+                                                randn(1, 2, 33, 20, dtype=torch.float32, seed=1)))
+    assert not isinstance(n, Exception)
+    same(p, n)
+
+
+@pytest.mark.parametrize("which", ["q", "k", "o", "row sums", "all", "size"])
+def test_attention_backward_refuses_mixed_saved_types(monkeypatch, which):
+    # tensors that the kernels would read by another type's width or size
+    f = lambda q, k: smooth_attn.sp2norm_flash_attention(q, k, k)
+    q, k = randn(1, 4, 33, 64), randn(1, 2, 33, 64, seed=1)
+
+    def call():
+        seen = []
+
+        def unpack(t):
+            name = ["q", "k", "v", "o", "row sums"][len(seen)]
+            seen.append(name)
+            if which == "size":
+                return t[:, :, :-1] if name == "k" else t
+            return t.half() if which in (name, "all") else t
+        return _hooked(f, unpack, q, k)
+    for got in both(monkeypatch, call)[:2]:
+        assert isinstance(got, ValueError), got
+
+
+def test_norm_backward_refuses_saved_x_of_another_size():
+    with pytest.raises(ValueError, match="grad_output's shape"):
+        _hooked(smooth_attn.softplus_norm_causal, lambda t: t[:1], randn(2, 16, 16))
+
+
 def test_transforms_and_subclasses(monkeypatch):
     x = randn(3, 16, 16)
     q = randn(2, 2, 16, 32)
