@@ -91,6 +91,18 @@ void check(int status, const char* what) {
                                  "): " + abi.status_string(status));
 }
 
+// Lets other Python threads run while a call allocates and launches, which may
+// wait: for a full queue, a first load of the kernel's code, an allocation that
+// frees cached memory first.  Gives the interpreter back before an exception
+// leaves its scope.
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    NoGil() = default;
+    NoGil(const NoGil&) = delete;
+    NoGil& operator=(const NoGil&) = delete;
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // ---------------------------------------------------------------------------
 // Which calls are ordinary.
 // ---------------------------------------------------------------------------
@@ -198,7 +210,10 @@ PyObject* py_norm_out(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!norm_input_ok(*x, causal) || out->scalar_type() != x->scalar_type() || out->device() != x->device() ||
         out->sizes() != x->sizes() || !out->is_contiguous())
         Py_RETURN_FALSE;
-    norm_fwd(*x, *out, causal, f);
+    {
+        const NoGil released;
+        norm_fwd(*x, *out, causal, f);
+    }
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -247,10 +262,16 @@ PyObject* py_causal_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor* x;
     if (n != 4 || !plain_mode() || !(x = plain(a[0])) || !f.parse(a[1], a[2], a[3]) || !norm_input_ok(*x, true))
         Py_RETURN_NONE;
-    if (at::GradMode::is_enabled() && x->requires_grad())
-        return THPVariable_Wrap(CausalNorm::apply(*x, f.alpha, f.theta, static_cast<int64_t>(f.power)));
-    Tensor y = at::empty_like(*x);
-    norm_fwd(*x, y, true, f);
+    Tensor y;
+    {
+        const NoGil released;
+        if (at::GradMode::is_enabled() && x->requires_grad()) {
+            y = CausalNorm::apply(*x, f.alpha, f.theta, static_cast<int64_t>(f.power));
+        } else {
+            y = at::empty_like(*x);
+            norm_fwd(*x, y, true, f);
+        }
+    }
     return THPVariable_Wrap(y);
     END_HANDLE_TH_ERRORS
 }
@@ -375,10 +396,16 @@ PyObject* py_flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
     else if (!as_double(a[3], c.scale))
         Py_RETURN_NONE;
     c.exact = a[5] == Py_True;
-    if (at::GradMode::is_enabled() && (q->requires_grad() || k->requires_grad() || v->requires_grad()))
-        return THPVariable_Wrap(Flash::apply(*q, *k, *v, c.scale, static_cast<int64_t>(c.window), c.exact));
-    Tensor o, row_sums;
-    flash_fwd(*q, *k, *v, c, o, row_sums);
+    Tensor o;
+    {
+        const NoGil released;
+        if (at::GradMode::is_enabled() && (q->requires_grad() || k->requires_grad() || v->requires_grad())) {
+            o = Flash::apply(*q, *k, *v, c.scale, static_cast<int64_t>(c.window), c.exact);
+        } else {
+            Tensor row_sums;
+            flash_fwd(*q, *k, *v, c, o, row_sums);
+        }
+    }
     return THPVariable_Wrap(o);
     END_HANDLE_TH_ERRORS
 }
@@ -421,18 +448,22 @@ PyObject* py_paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
         scale = 1.0 / std::sqrt(static_cast<double>(D));
     else if (!as_double(a[5], scale))
         Py_RETURN_NONE;
-    Tensor out = at::empty({B, Hq, D}, q->options().dtype(at::kBFloat16).requires_grad(false));
-    const int b = static_cast<int>(B), hq = static_cast<int>(Hq), d = static_cast<int>(D);
-    const int max_pages = static_cast<int>(table->size(1));
-    const int64_t ws_bytes = abi.paged_decode_workspace_size(b, hq, d, max_pages, block_size);
-    Tensor ws = at::empty({std::max<int64_t>(1, (ws_bytes + 3) / 4)}, out.options().dtype(at::kFloat));
-    const c10::DeviceGuard guard(q->device());
-    check(abi.paged_decode(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), table->data_ptr<int32_t>(),
-                           lens->data_ptr<int32_t>(), b, hq, static_cast<int>(Hkv), d, block_size, max_pages,
-                           static_cast<int>(k->size(0)), strides(*q), strides(*k), strides(*v), strides(out),
-                           table->stride(0), static_cast<float>(scale), mixed ? SA_PAGED_DTYPES(qc, kc) : qc,
-                           ws.data_ptr<float>(), ws.numel() * 4, stream_of(*q)),
-          "sa_paged_decode");
+    Tensor out;
+    {
+        const NoGil released;
+        out = at::empty({B, Hq, D}, q->options().dtype(at::kBFloat16).requires_grad(false));
+        const int b = static_cast<int>(B), hq = static_cast<int>(Hq), d = static_cast<int>(D);
+        const int max_pages = static_cast<int>(table->size(1));
+        const int64_t ws_bytes = abi.paged_decode_workspace_size(b, hq, d, max_pages, block_size);
+        Tensor ws = at::empty({std::max<int64_t>(1, (ws_bytes + 3) / 4)}, out.options().dtype(at::kFloat));
+        const c10::DeviceGuard guard(q->device());
+        check(abi.paged_decode(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), table->data_ptr<int32_t>(),
+                               lens->data_ptr<int32_t>(), b, hq, static_cast<int>(Hkv), d, block_size, max_pages,
+                               static_cast<int>(k->size(0)), strides(*q), strides(*k), strides(*v), strides(out),
+                               table->stride(0), static_cast<float>(scale), mixed ? SA_PAGED_DTYPES(qc, kc) : qc,
+                               ws.data_ptr<float>(), ws.numel() * 4, stream_of(*q)),
+              "sa_paged_decode");
+    }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
@@ -454,15 +485,19 @@ PyObject* py_paged_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!paging_ok(*k, B, Hkv, D, block_size, *k, *v, *table, *lens) || D % (16 / k->element_size()) != 0 ||
         !operand_ok(*kn) || !operand_ok(*vn) || kn->strides() != vn->strides() || B > INT32_MAX || n_new > INT32_MAX)
         Py_RETURN_NONE;
-    const c10::DeviceGuard guard(k->device());
-    Tensor out = at::empty(lens->sizes(), lens->options());
-    check(abi.paged_kv_append_lens(kn->data_ptr(), vn->data_ptr(), k->data_ptr(), v->data_ptr(),
-                                   table->data_ptr<int32_t>(), lens->data_ptr<int32_t>(), out.data_ptr<int32_t>(),
-                                   lens->numel(), static_cast<int>(B), static_cast<int>(Hkv),
-                                   static_cast<int>(n_new), static_cast<int>(D), block_size,
-                                   static_cast<int>(table->size(1)), static_cast<int>(k->size(0)), strides(*kn),
-                                   strides(*k), strides(*v), table->stride(0), code, stream_of(*k)),
-          "sa_paged_kv_append_lens");
+    Tensor out;
+    {
+        const NoGil released;
+        const c10::DeviceGuard guard(k->device());
+        out = at::empty(lens->sizes(), lens->options());
+        check(abi.paged_kv_append_lens(kn->data_ptr(), vn->data_ptr(), k->data_ptr(), v->data_ptr(),
+                                       table->data_ptr<int32_t>(), lens->data_ptr<int32_t>(), out.data_ptr<int32_t>(),
+                                       lens->numel(), static_cast<int>(B), static_cast<int>(Hkv),
+                                       static_cast<int>(n_new), static_cast<int>(D), block_size,
+                                       static_cast<int>(table->size(1)), static_cast<int>(k->size(0)), strides(*kn),
+                                       strides(*k), strides(*v), table->stride(0), code, stream_of(*k)),
+              "sa_paged_kv_append_lens");
+    }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }

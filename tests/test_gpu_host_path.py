@@ -346,6 +346,56 @@ def test_norm_backward_refuses_saved_x_of_another_size():
         _hooked(smooth_attn.softplus_norm_causal, lambda t: t[:1], randn(2, 16, 16))
 
 
+@pytest.mark.parametrize("entry", ["norm_out", "causal_norm", "causal_norm grad", "flash", "flash grad", "paged",
+                                   "paged_append"])
+def test_other_python_threads_run_during_a_launch(entry):
+    # a launch that waits (a full queue, a first load of its code) must not stop
+    # the interpreter.  In place of every launch the path calls PyGILState_Check,
+    # whose 1 (this thread holds the interpreter) is an error status here.
+    import ctypes
+
+    addr = {n: ctypes.cast(getattr(_lib.load(), n), ctypes.c_void_p).value for n in _lib.SIGNATURES}
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    launches = ("sa_norm_fwd", "sa_norm_bwd", "sa_flash_fwd", "sa_flash_bwd_ws", "sa_paged_decode",
+                "sa_paged_kv_append_lens")
+    x, q, k = randn(2, 32, 32), randn(1, 4, 40, 64), randn(1, 2, 40, 64)
+    cache = torch.zeros(4, 2, 16, 64, device=DEV, dtype=torch.bfloat16)
+    table = torch.zeros(1, 4, device=DEV, dtype=torch.int32)
+    lens = torch.ones(1, device=DEV, dtype=torch.int32)
+    host = _lib.host()
+    host.bind({**addr, **{n: check for n in launches}})
+    try:
+        if entry == "norm_out":
+            assert host.norm_out(torch.empty_like(x), x, True, 2.0, 0.5, 2)
+        elif entry.startswith("causal_norm"):
+            y = host.causal_norm(x.requires_grad_("grad" in entry), 2.0, 0.5, 2)
+            if y.requires_grad:
+                y.sum().backward()
+        elif entry.startswith("flash"):
+            o = host.flash(q.requires_grad_("grad" in entry), k, k, None, 0, False)
+            if o.requires_grad:
+                o.sum().backward()
+        elif entry == "paged":
+            assert host.paged(q[:, :, :1], cache, cache, table, lens, None, 16) is not None
+        else:
+            new = k[:, :, :1].contiguous()
+            assert host.paged_append(cache, cache, new, new, table, lens, 16) is not None
+    finally:
+        host.bind(addr)
+
+
+def test_errors_of_hooks_and_allocations_reach_the_caller():
+    q, k = randn(1, 4, 40, 64), randn(1, 2, 40, 64)
+
+    def pack(t):
+        raise KeyError("from the hook")
+    for fn in (lambda: smooth_attn.sp2norm_flash_attention(q.clone().requires_grad_(True), k, k),
+               lambda: smooth_attn.softplus_norm_causal(q[..., :40].clone().requires_grad_(True))):
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), pytest.raises(KeyError, match="from the hook"):
+            fn()
+    same(smooth_attn.sp2norm_flash_attention(q, k, k), smooth_attn.sp2norm_flash_attention(q.clone(), k, k))
+
+
 def test_transforms_and_subclasses(monkeypatch):
     x = randn(3, 16, 16)
     q = randn(2, 2, 16, 32)
