@@ -231,6 +231,22 @@ int sa_flash_bwd_ws(const void* q, const void* k, const void* v, const void* o,
                     sa_stream_t stream);
 
 /*
+ * Which builds the attention launches choose at head dims up to 128 (host
+ * arithmetic only, no launch).
+ * sa_flash_fwd_key_split: waves that share a query tile (1, 2 or 4) in
+ * sa_flash_fwd, sa_flash_rope_fwd and sa_flash_fp8_fwd, for K and V rows at
+ * most kv_row_bytes apart.
+ * sa_flash_bwd_plan: plan[0], plan[1] = row groups per block (1 or 2) of the
+ * dQ and the dK/dV kernel, plan[2] = query-range splits, of a 16-bit
+ * sa_flash_bwd_ws with workspace_bytes of workspace.
+ */
+int sa_flash_fwd_key_split(int B, int Hq, int Hkv, int T, int D,
+                           int window_size, int exact_math,
+                           int64_t kv_row_bytes);
+int sa_flash_bwd_plan(int B, int Hq, int Hkv, int T, int D, int window_size,
+                      int exact_math, int64_t workspace_bytes, int* plan);
+
+/*
  * Per-tensor absmax quantisation to float8_e4m3fn, entirely on the device:
  *   scale = max(amax|x| / 448, 1e-12);  x8 = e4m3fn(clamp(x / scale, +-448))
  * x: n contiguous elements of dtype (SA_F32/SA_F16/SA_BF16); x8: n bytes.

@@ -965,6 +965,13 @@ BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, in
 }
 
 constexpr int kMaxSplit = 16;
+// The most splits (a power of two) whose partials fit the workspace.
+int splits_that_fit(int B, int Hkv, int T, int dr, int64_t workspace_bytes) {
+    int n = workspace_bytes > 0 ? kMaxSplit : 1;
+    while (n > 1 && bwd_part_bytes(n, B, Hkv, T, dr) > workspace_bytes) n /= 2;
+    return n;
+}
+
 BwdPlan choose_bwd_plan(int B, int Hkv, int T, int G, int W, int dr, int max_split, bool groups) {
     const int64_t blocks = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv;
     if (blocks >= 8 * kBwdXcdSlots * 8 || blocks == 0) return BwdPlan{};  // full grids
@@ -991,6 +998,20 @@ extern "C" int64_t sa_flash_bwd_workspace_size(int B, int Hq, int Hkv, int T, in
     // (exact square roots, which have no groups, may then split)
     const bool small = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv < 64;
     return bwd_part_bytes(small ? std::max(n_split, 2) : n_split, B, Hkv, T, D);
+}
+
+extern "C" int sa_flash_bwd_plan(int B, int Hq, int Hkv, int T, int D, int window_size, int exact_math,
+                                 int64_t workspace_bytes, int* plan) {
+    using namespace sa;
+    if (!plan) return SA_ERR_NULL_POINTER;
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || Hq % Hkv != 0 || window_size < 0) return SA_ERR_BAD_SHAPE;
+    if (D < 8 || D > 128 || D % 8 != 0) return SA_ERR_UNSUPPORTED;
+    const BwdPlan p = choose_bwd_plan(B, Hkv, T, Hq / Hkv, window_size, D,
+                                      splits_that_fit(B, Hkv, T, D, workspace_bytes), !exact_math);
+    plan[0] = p.dq_groups;
+    plan[1] = p.kv_groups;
+    plan[2] = p.n_split;
+    return 0;
 }
 
 extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -1061,13 +1082,10 @@ extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, cons
     prm.dr = D;
     prm.scale = scale;
     // the plan among the split counts whose partials fit the workspace
-    int max_split = 1;
-    if (workspace && workspace_bytes > 0) {
-        if (!aligned16(workspace)) return SA_ERR_BAD_STRIDE;
-        max_split = kMaxSplit;
-        while (max_split > 1 && bwd_part_bytes(max_split, B, Hkv, T, D) > workspace_bytes) max_split /= 2;
-    }
-    const BwdPlan plan = choose_bwd_plan(B, Hkv, T, prm.G, window_size, D, max_split, !exact_math);
+    if (!workspace) workspace_bytes = 0;
+    if (workspace_bytes > 0 && !aligned16(workspace)) return SA_ERR_BAD_STRIDE;
+    const BwdPlan plan = choose_bwd_plan(B, Hkv, T, prm.G, window_size, D,
+                                         splits_that_fit(B, Hkv, T, D, workspace_bytes), !exact_math);
     prm.n_split = plan.n_split;
     prm.part = plan.n_split > 1 ? static_cast<float*>(workspace) : nullptr;
     // the block order's group sizes, worked out here rather than before every block's first load

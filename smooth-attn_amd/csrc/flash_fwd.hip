@@ -212,6 +212,17 @@ bool strides_ok(const int64_t* s, int elem_bytes) {
     return s[3] == 1 && s[0] % a == 0 && s[1] % a == 0 && s[2] % a == 0;
 }
 
+void set_sizes(FlashParams& prm, int B, int Hq, int Hkv, int T, int D, int window_size) {
+    prm.B = B;
+    prm.Hq = Hq;
+    prm.Hkv = Hkv;
+    prm.T = T;
+    prm.G = Hq / Hkv;
+    prm.window = window_size;
+    prm.dr = D;
+    set_grid(prm, Split<1>::BQ);
+}
+
 int fill_params(FlashParams& prm, const void* q, const void* k, const void* v, void* o, float* row_sums, int B,
                 int Hq, int Hkv, int T, int D, const int64_t* q_strides, const int64_t* k_strides,
                 const int64_t* v_strides, const int64_t* o_strides, float scale, int window_size, int qk_bytes,
@@ -236,20 +247,27 @@ int fill_params(FlashParams& prm, const void* q, const void* k, const void* v, v
         prm.vs[i] = v_strides[i];
         prm.os[i] = o_strides[i];
     }
-    prm.B = B;
-    prm.Hq = Hq;
-    prm.Hkv = Hkv;
-    prm.T = T;
-    prm.G = Hq / Hkv;
-    prm.window = window_size;
-    set_grid(prm, Split<1>::BQ);
-    prm.dr = D;
+    set_sizes(prm, B, Hq, Hkv, T, D, window_size);
     prm.scale = scale;
     return 0;
 }
 
 }  // namespace
 }  // namespace sa
+
+extern "C" int sa_flash_fwd_key_split(int B, int Hq, int Hkv, int T, int D, int window_size, int exact_math,
+                                      int64_t kv_row_bytes) {
+    using namespace sa;
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || Hq % Hkv != 0 || window_size < 0 || kv_row_bytes <= 0 ||
+        kv_row_bytes > kMaxRowStrideBytes)
+        return SA_ERR_BAD_SHAPE;
+    if (D < 8 || D > 128 || D % 8 != 0) return SA_ERR_UNSUPPORTED;
+    if (exact_math) return 1;
+    FlashParams prm{};
+    set_sizes(prm, B, Hq, Hkv, T, D, window_size);
+    prm.ks[2] = prm.vs[2] = kv_row_bytes;
+    return key_split_for(prm, 1, 1);
+}
 
 extern "C" int sa_flash_fwd(const void* q, const void* k, const void* v, void* o, float* row_sums, int B, int Hq,
                             int Hkv, int T, int D, const int64_t* q_strides, const int64_t* k_strides,

@@ -65,6 +65,8 @@ SIGNATURES = {
                                 c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, _I64P, _I64P, _I64P,
                                 _I64P, _I64P, _I64P, _I64P, _I64P, c_float, c_int, c_int, c_int, c_void_p, c_int64,
                                 c_void_p]),
+    "sa_flash_fwd_key_split": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64]),
+    "sa_flash_bwd_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64, POINTER(c_int)]),
     "sa_fp8_quantize": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p]),
     "sa_fp8_quantize_many": (c_int, [c_int, POINTER(c_void_p), POINTER(c_void_p), _I64P, c_int,
                                      c_void_p, c_void_p, c_void_p]),

@@ -219,6 +219,28 @@ def test_flash_bwd_workspace_size():
     assert st == -5
 
 
+def test_attention_build_queries():
+    # host arithmetic: invalid sizes are refused, full grids and exact square
+    # roots take the plain builds, a short grid does not, whatever its dtype;
+    # splits need a workspace that holds their partials
+    lib, plan = _lib.load(), (ctypes.c_int * 3)()
+    split = lib.sa_flash_fwd_key_split
+    assert split(1, 4, 3, 512, 128, 0, 0, 256) == -2 and split(1, 4, 2, 512, 128, -1, 0, 256) == -2
+    assert split(1, 4, 2, 512, 132, 0, 0, 256) == -6 and split(1, 4, 2, 512, 128, 0, 0, 1 << 25) == -2
+    assert split(8, 32, 32, 8192, 128, 0, 0, 256) == 1
+    assert split(1, 4, 2, 512, 128, 0, 0, 256) == 4 and split(1, 4, 2, 512, 128, 0, 1, 256) == 1
+    assert split(1, 4, 2, 512, 128, 0, 0, (1 << 23) + 16) == 2  # 128-row tiles bound the row stride
+    query = lib.sa_flash_bwd_plan
+    assert query(1, 4, 2, 512, 128, 0, 0, 0, None) == -1
+    assert query(1, 4, 3, 512, 128, 0, 0, 0, plan) == -2 and query(1, 4, 2, 512, 256, 0, 0, 0, plan) == -6
+    assert query(8, 32, 32, 8192, 128, 0, 0, 1 << 40, plan) == 0 and list(plan) == [1, 1, 1]
+    assert query(1, 8, 1, 16384, 128, 0, 0, 0, plan) == 0 and plan[2] == 1
+    ws = lib.sa_flash_bwd_workspace_size(1, 8, 1, 16384, 128, 0, _lib.SA_BF16)
+    assert query(1, 8, 1, 16384, 128, 0, 0, ws, plan) == 0 and plan[2] > 1
+    n = plan[2]
+    assert query(1, 8, 1, 16384, 128, 0, 0, ws - 16, plan) == 0 and 1 <= plan[2] < n
+
+
 def test_paged_decode_head_dims():
     # D must be a multiple of 8 in 8..1024 (8..512 over caches read as bf16
     # hi + lo tiles: fp32, or fp16 under an fp32 q); checked before any HIP call

@@ -2,13 +2,14 @@
 merged in LDS): grids too short to fill the GPU take them, alone or with the
 dK/dV split.  Lengths around tile and block edges, windows, GQA, padded head
 dims, strided inputs; against float64 gradients."""
+import ctypes
 import math
 
 import pytest
 import torch
 
 from oracle import eager
-from smooth_attn import kernels
+from smooth_attn import _lib, kernels
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -17,6 +18,14 @@ DEV = "cuda"
 def rel_err(got, ref):
     got, ref = got.detach().double().cpu(), ref.detach().double().cpu()
     return float((got - ref).abs().max() / ref.abs().max().clamp(min=1e-30))
+
+
+def plan(B, Hq, Hkv, T, D, window, exact=0):
+    """(dQ groups, dK/dV groups, splits) of the backward's launch."""
+    lib, out = _lib.load(), (ctypes.c_int * 3)()
+    ws = lib.sa_flash_bwd_workspace_size(B, Hq, Hkv, T, D, window, _lib.SA_BF16)
+    assert lib.sa_flash_bwd_plan(B, Hq, Hkv, T, D, window, exact, ws, out) == 0
+    return tuple(out)
 
 
 def grads64(q, k, v, o, do, window):
@@ -36,6 +45,9 @@ def grads64(q, k, v, o, do, window):
     (1, 16, 4, 577, 64, 0), (1, 8, 2, 1025, 128, 0), (1, 8, 8, 900, 128, 130), (1, 8, 2, 800, 64, 65),
     (1, 4, 4, 1100, 128, 1), (1, 16, 2, 600, 80, 333)])
 def test_groups_match_float64(dtype, B, Hq, Hkv, T, D, window):
+    # (a window of 1 leaves the dQ blocks, and at D = 128 the dK/dV blocks, nothing to share)
+    dq_groups, kv_groups, _ = plan(B, Hq, Hkv, T, D, window)
+    assert (kv_groups == 2) == (window != 1) and (dq_groups == 2 or 0 < window <= 130)
     g = torch.Generator().manual_seed(T + D)
     mk = lambda H: torch.randn(B, T, H, D, generator=g).to(dtype).transpose(1, 2)  # rows of all heads side by side
     q, k, v, do = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
@@ -55,6 +67,7 @@ def test_groups_match_float64(dtype, B, Hq, Hkv, T, D, window):
 
 def test_exact_square_roots_keep_one_group():
     # (no two-group build): same gradients as the fast build within rounding
+    assert plan(1, 8, 8, 700, 64, 0)[:2] == (2, 2) and plan(1, 8, 8, 700, 64, 0, 1)[:2] == (1, 1)
     g = torch.Generator().manual_seed(1)
     q, k, v, do = (torch.randn(1, 8, 700, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
     o, rs = kernels._sp2norm_flash_fwd(q, k, v, 0.125, 1, 0)

@@ -10,11 +10,17 @@ import torch
 
 import smooth_attn
 from oracle import eager
-from smooth_attn import kernels
+from smooth_attn import _lib, kernels
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 TWO, FOUR = (2, 32, 8), (1, 4, 2)  # (B, Hq, Hkv) of grids that take 2 and 4 key groups at the lengths below
+GROUPS = {TWO: 2, FOUR: 4}
+
+
+def takes(heads, T, D, window, groups):
+    """The launch takes the build with this many key groups (rows of D 16-bit elements, heads side by side)."""
+    return _lib.load().sa_flash_fwd_key_split(*heads, T, D, window, 0, 2 * D * heads[2]) == groups
 
 
 def rel_err(got, ref):
@@ -46,21 +52,25 @@ def check(q, k, v, window):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,T,D,window", [
     (FOUR, 256, 128, 0), (FOUR, 257, 128, 0), (FOUR, 319, 64, 0), (FOUR, 385, 32, 0), (FOUR, 511, 128, 1),
-    (FOUR, 640, 128, 33), (FOUR, 641, 96, 200), (FOUR, 1023, 128, 0), (FOUR, 1100, 40, 129), (FOUR, 2049, 64, 600),
+    (FOUR, 640, 128, 33), (FOUR, 640, 128, 192), (FOUR, 641, 96, 200), (FOUR, 1023, 128, 0), (FOUR, 1100, 40, 129), (FOUR, 2049, 64, 600),
     (TWO, 385, 128, 0), (TWO, 449, 64, 0), (TWO, 511, 32, 0), (TWO, 512, 128, 300), (TWO, 513, 72, 0),
     (TWO, 500, 128, 450)])
 def test_key_split_matches_oracle(dtype, heads, T, D, window):
+    # (a window of 33 leaves blocks of 640 rows too little to share out four ways)
+    assert takes(heads, T, D, window, 2 if (heads, T, window) == (FOUR, 640, 33) else GROUPS[heads])
     check(*qkv(heads, T, D, dtype, T + D), window)
 
 
 @pytest.mark.parametrize("heads,T", [(FOUR, 300), (TWO, 500)])
 def test_key_split_of_strided_inputs(heads, T):
+    assert takes(heads, T, 128, 0, GROUPS[heads])
     check(*qkv(heads, T, 128, torch.bfloat16, 5, bthd=True), 0)
 
 
 @pytest.mark.parametrize("heads,T,D", [(FOUR, 333, 128), (FOUR, 700, 64), (TWO, 511, 32)])
 @pytest.mark.parametrize("v8", [True, False])
 def test_key_split_fp8(heads, T, D, v8):
+    assert takes(heads, T, D, 0, GROUPS[heads])
     q, k, v = qkv(heads, T, D, torch.bfloat16, T)
     (q8, qs), (k8, ks), (v8t, vs) = (eager.quantize_to_fp8(t) for t in (q, k, v))
     vv, vsc = (v8t, vs) if v8 else (v, 1.0)
@@ -75,6 +85,7 @@ def test_key_split_fp8(heads, T, D, v8):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,T,D", [(FOUR, 333, 128), (TWO, 511, 64)])
 def test_key_split_rope(dtype, heads, T, D):
+    assert takes(heads, T, D, 0, GROUPS[heads])
     q, k, v = qkv(heads, T, D, dtype, T + 1)
     cos, sin = smooth_attn.precompute_rope_cos_sin(D, T, device="cpu")
     o = smooth_attn.sp2norm_rope_flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), cos.to(DEV), sin.to(DEV))

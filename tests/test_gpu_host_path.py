@@ -182,18 +182,27 @@ def test_paged_forms(monkeypatch, qd, cd, D):
     forms = [caches(), [c.transpose(1, 2).contiguous().transpose(1, 2) for c in caches()]]
     if cd != torch.float8_e4m3fn:
         forms.append([torch.cat([c, c], -1)[..., :D] for c in caches()])
+    # taken: one type for all (or bf16 q over e4m3fn caches), head dims of whole
+    # 16-byte rows, int32 paging with unit strides
+    pair = qd == cd or (qd, cd) == (torch.bfloat16, torch.float8_e4m3fn)
+    row16 = 16 if cd == torch.float8_e4m3fn else 8
     for k, v in forms:
         for t, n in ((table.int(), lens.int()), (table, lens), (table.int().t().contiguous().t(), lens.int()),
                      (table.int(), torch.stack([lens.int(), lens.int()], 1)[:, 0])):
+            paging = t.dtype == torch.int32 and t.stride(1) == 1 and n.dtype == torch.int32 and n.is_contiguous()
             q = randn(B, 4, 1, D, dtype=qd, seed=4)
             for qq in (q, randn(B, 1, 4, D, dtype=qd, seed=4).transpose(1, 2)):
-                same(*both(monkeypatch, lambda: smooth_attn.sp2norm_paged_attention(qq, k, v, t, n))[:2])
+                p, nat, took = both(monkeypatch, lambda: smooth_attn.sp2norm_paged_attention(qq, k, v, t, n))
+                same(p, nat)
+                assert took == (pair and paging and D % row16 == 0)
             for new in (randn(B, Hkv, 2, D, seed=5), randn(B, 2, Hkv, D, seed=5).transpose(1, 2)):
                 def append():
                     kk, vv = k.clone(memory_format=torch.preserve_format), v.clone(memory_format=torch.preserve_format)
                     nn = new.to(cd)
                     return [smooth_attn.sp2norm_paged_kv_append(kk, vv, nn, nn, t, n), kk, vv]
-                same(*both(monkeypatch, append)[:2])
+                p, nat, took = both(monkeypatch, append)
+                same(p, nat)
+                assert took == (paging and D % row16 == 0)
 
 
 def _train(x):
