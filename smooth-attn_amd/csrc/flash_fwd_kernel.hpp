@@ -606,11 +606,15 @@ __global__ __launch_bounds__(kThreads, KS == 2 && D == 64 ? 4 : 1) void flash_fw
     // last row).  Separate loops per kind keep the accumulators in fixed
     // registers.  Waves whose rows all lie past T only keep the barriers.
     // With two query tiles, the span runs from the first tile's first row
-    // (wf) to the last tile's last row (wl).
+    // (wf) to the last tile's last row (wl).  With 128-key tiles (KS = 4) a
+    // wave counts the tiles whose 64 keys around its part see some row: an Inf
+    // or NaN of V (times a weight of 0) then reaches the rows that it reaches
+    // under every key split.
     const int wf = wq0[0], wl = wq0[kQT - 1] + 31;
+    const int part0 = KS == 4 ? (grp >> 1) * 64 : 0;  // first of those keys in the tile
     int t_first = kv_begin;
-    if (W > 0 && wf - W + 1 > 0) t_first = max(t_first, (wf - W + 1) / kBKV);
-    const int t_last = wf < T_ ? min(wl / kBKV, kv_end - 1) : t_first - 1;
+    if (W > 0 && wf - W + 1 > 0) t_first = max(t_first, (wf - W + 1 + kBKV - 64 - part0) / kBKV);
+    const int t_last = wf < T_ ? min((wl - part0) >> (KS == 4 ? 7 : 6), kv_end - 1) : t_first - 1;
     int ja = t_first;
     if (W > 0 && wl - W >= 0) ja = max(ja, (wl - W) / kBKV + 1);
     const int jb = (wf + 1) / kBKV;

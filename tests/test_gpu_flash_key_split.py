@@ -91,3 +91,25 @@ def test_key_split_rope(dtype, heads, T, D):
     o = smooth_attn.sp2norm_rope_flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), cos.to(DEV), sin.to(DEV))
     ref = eager.rope_flash_attention_eager(q.double(), k.double(), v.double(), cos, sin, round_to=dtype)
     assert rel_err(o, ref) <= 1e-2
+
+
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+@pytest.mark.parametrize("heads,T,D,window", [
+    (FOUR, 640, 128, 0), (FOUR, 577, 64, 0), (FOUR, 640, 128, 192), (FOUR, 641, 96, 200), (FOUR, 300, 32, 0),
+    (TWO, 449, 64, 0), (TWO, 512, 128, 300)])
+def test_non_finite_values_reach_the_same_rows_in_every_build(heads, T, D, window, bad):
+    # 0 x Inf: a bad V row reaches rows that do not see its key where a wave
+    # walks the key's tile.  The build without a key split (exact square
+    # roots have no other) walks tiles of 64 keys.
+    assert takes(heads, T, D, window, GROUPS[heads])
+    q, k, v = (t.to(DEV) for t in qkv(heads, T, D, torch.bfloat16, 7))
+    clean = smooth_attn.sp2norm_flash_attention(q, k, v, window_size=window)
+    for key in (70, 127, 128, 191, 255, T - 40):
+        vb = v.clone()
+        vb[:, :, key, 3] = bad
+        o = smooth_attn.sp2norm_flash_attention(q, k, vb, window_size=window)
+        one = smooth_attn.sp2norm_flash_attention(q, k, vb, window_size=window, exact_math=True)
+        hit = ~torch.isfinite(o)
+        assert torch.equal(hit, ~torch.isfinite(one)), key
+        assert torch.equal(o[~hit], clean[~hit])
+        assert bool(hit[:, :, key, 3].all()) and not bool(hit[:, :, : key // 64 * 64].any())
