@@ -28,6 +28,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include <cmath>
 #include <cstring>
@@ -523,4 +524,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native call path (see csr
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&module);
+    // (the tensors' layout in memory is that torch's)
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_void_p
 from pathlib import Path
 
@@ -122,26 +123,55 @@ def load():
         return lib
 
 
+class NothingOrdinary:
+    """The native call path's answers where it takes no call."""
+
+    @staticmethod
+    def _none(*_):
+        return None
+
+    norm_out = causal_norm = flash = paged = paged_append = _none
+
+
+def _load_host(lib):
+    """The extension of csrc/host/host.cpp, bound to the library's functions."""
+    if not _HOST_PATH.exists():
+        raise ImportError(f"{_HOST_PATH} not found")
+    import importlib.util
+
+    import torch
+
+    spec = importlib.util.spec_from_file_location(f"{__package__}._host", _HOST_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    if mod.torch_version != torch.__version__.split("+")[0]:
+        raise ImportError(f"{_HOST_PATH} was built against torch {mod.torch_version}, not {torch.__version__}")
+    mod.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
+    return mod
+
+
 def host():
-    """The native call path (csrc/host/host.cpp), loaded once and bound to the
-    library's functions."""
+    """The native call path, loaded once.  Every call that it takes has a Python
+    path with the same kernels and results, so where the extension is missing
+    or does not fit the installed torch, a warning says so once and it takes
+    none; without the library it takes none either, and the Python path raises
+    after its argument checks."""
     global _host
     if _host is not None:
         return _host
-    lib = load()
+    try:
+        lib = load()
+    except (OSError, RuntimeError):
+        return NothingOrdinary
     with _lock:
-        if _host is not None:
-            return _host
-        if not _HOST_PATH.exists():
-            raise RuntimeError(f"smooth_attn host extension not found at {_HOST_PATH}; {_BUILD}")
-        import importlib.util
-
-        spec = importlib.util.spec_from_file_location(f"{__package__}._host", _HOST_PATH)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
-        mod.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
-        _host = mod
-        return mod
+        if _host is None:
+            try:
+                _host = _load_host(lib)
+            except (ImportError, OSError) as e:
+                _host = NothingOrdinary
+                warnings.warn(f"smooth_attn: native call path not available ({e}); small calls cost more host time "
+                              f"until it is built: {_BUILD}", RuntimeWarning, stacklevel=3)
+        return _host
 
 
 def check(status: int, what: str) -> None:

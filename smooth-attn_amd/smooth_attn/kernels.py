@@ -107,16 +107,6 @@ def _resolve_family(alpha, theta, power, family):
     return family
 
 
-class _NothingOrdinary:
-    """The native call path's answers where no tensor can be on a GPU."""
-
-    @staticmethod
-    def _none(*_):
-        return None
-
-    norm_out = causal_norm = flash = paged = paged_append = _none
-
-
 def _native():
     """The native call path (csrc/host/host.cpp).  It takes the calls whose
     tensors the kernels can use as they are and answers None (or False) to
@@ -124,7 +114,7 @@ def _native():
     CUDA is initialised no tensor is on a GPU and no call is ordinary: the
     libraries are not loaded for it, and the Python path's checks refuse it."""
     if _lib._host is None and not torch.cuda.is_initialized():
-        return _NothingOrdinary
+        return _lib.NothingOrdinary
     return _lib.host()
 
 
