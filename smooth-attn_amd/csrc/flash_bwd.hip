@@ -993,11 +993,13 @@ extern "C" int64_t sa_flash_bwd_workspace_size(int B, int Hq, int Hkv, int T, in
     if (dtype != SA_BF16 && dtype != SA_F16) return 0;
     if (B == 0 || T == 0 || D > 512) return 0;
     if (D > 128) return flash_bwd_wide_workspace_size(B, Hq, Hkv, T, D, window_size);
-    const int n_split = choose_bwd_plan(B, Hkv, T, Hq / Hkv, window_size, D, kMaxSplit, true).n_split;
-    // room for two splits in the smallest grids, also where none is chosen
-    // (exact square roots, which have no groups, may then split)
-    const bool small = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv < 64;
-    return bwd_part_bytes(small ? std::max(n_split, 2) : n_split, B, Hkv, T, D);
+    // room for the plans with and without groups (exact square roots have none, and then split more), and for
+    // two splits in the smallest grids, also where none is chosen
+    const int G = Hq / Hkv;
+    int n_split = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv < 64 ? 2 : 1;
+    for (const bool groups : {true, false})
+        n_split = std::max(n_split, choose_bwd_plan(B, Hkv, T, G, window_size, D, kMaxSplit, groups).n_split);
+    return bwd_part_bytes(n_split, B, Hkv, T, D);
 }
 
 extern "C" int sa_flash_bwd_plan(int B, int Hq, int Hkv, int T, int D, int window_size, int exact_math,
