@@ -886,11 +886,16 @@ struct BwdCosts {
     double dq_setup[2], dq_alone, dq_tile[2], dq_share_setup[2], dq_share[2], dq_ragged;
     double kv_setup, kv_alone, kv_iter[2], kv_share_setup[2], kv_share[2], kv_ragged;
     double part_tb_s, part_setup;
+    double exact_iter;  // an iteration with exact square roots, times the above
 };
+// Exact square roots (one group always), fitted to 80 shapes of the same
+// ranges: the choice averages 0.6% over the fastest S, without the factors
+// 1.8% and at worst 20% ([2,12,1280,128]: S = 1 / 2 / 4 151 / 135 / 143 us).
+constexpr double kExactPart = 0.7;  // their part of part_setup
 constexpr BwdCosts kBwdCosts128 = {{3.5, 10.7}, 2.14, {2.43, 0.89}, {6.8, 5.7}, {0.43, 1.74}, 0.41,
-                                   6.4, 2.79, {3.33, 2.72}, {7.0, 9.9}, {1.85, 2.53}, 0.05, 8.0, 14.3};
+                                   6.4, 2.79, {3.33, 2.72}, {7.0, 9.9}, {1.85, 2.53}, 0.05, 8.0, 14.3, 1.6};
 constexpr BwdCosts kBwdCosts64 = {{3.7, 10.5}, 2.02, {1.88, 0.96}, {5.7, 8.0}, {1.06, 1.63}, 0.09,
-                                  12.5, 2.59, {2.59, 1.54}, {3.3, 10.2}, {1.59, 2.42}, 0.38, 5.0, 4.2};
+                                  12.5, 2.59, {2.59, 1.54}, {3.3, 10.2}, {1.59, 2.42}, 0.38, 5.0, 4.2, 1.3};
 
 struct BwdPlan {
     int dq_groups = 1, kv_groups = 1, n_split = 1;
@@ -904,7 +909,13 @@ double with_ragged_end(double longest, double shared, double ragged) {
 // blocks of two groups may be used (exact square roots have none).
 BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, int max_split, bool groups) {
     constexpr double kCus = 256.0;
-    const BwdCosts& c = bwd_kernel_d(dr) == 128 ? kBwdCosts128 : kBwdCosts64;
+    BwdCosts c = bwd_kernel_d(dr) == 128 ? kBwdCosts128 : kBwdCosts64;
+    if (!groups) {
+        c.kv_alone *= c.exact_iter;
+        c.kv_iter[0] *= c.exact_iter;
+        c.kv_share[0] *= c.exact_iter;
+        c.part_setup *= kExactPart;
+    }
     const int nkb = (T + kBwdBK - 1) / kBwdBK, nqb = (T + kBwdBQ - 1) / kBwdBQ;
     const int n_kv = (T + kBwdKT - 1) / kBwdKT;
     int64_t kv_sum = 0, dq_sum = 0;

@@ -241,6 +241,22 @@ def test_attention_build_queries():
     assert query(1, 8, 1, 16384, 128, 0, 0, ws - 16, plan) == 0 and 1 <= plan[2] < n
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T,D,window", [
+    (4, 32, 8, 512, 64, 128), (1, 32, 32, 1024, 64, 0), (1, 32, 8, 2048, 128, 0), (1, 8, 8, 4096, 128, 0),
+    (2, 16, 16, 1024, 32, 0), (8, 32, 8, 300, 64, 0), (2, 12, 12, 1280, 128, 0), (1, 4, 4, 314, 96, 0)])
+def test_exact_backward_gets_the_workspace_of_its_splits(B, Hq, Hkv, T, D, window):
+    # exact square roots have no two-group blocks and split where the fast
+    # build need not: the workspace that callers are told to bring holds both
+    lib = _lib.load()
+    ws = lib.sa_flash_bwd_workspace_size(B, Hq, Hkv, T, D, window, _lib.SA_BF16)
+    for exact in (0, 1):
+        told, free = (ctypes.c_int * 3)(), (ctypes.c_int * 3)()
+        assert lib.sa_flash_bwd_plan(B, Hq, Hkv, T, D, window, exact, ws, told) == 0
+        assert lib.sa_flash_bwd_plan(B, Hq, Hkv, T, D, window, exact, 1 << 40, free) == 0
+        assert list(told) == list(free)
+    assert told[2] > 1
+
+
 def test_paged_decode_head_dims():
     # D must be a multiple of 8 in 8..1024 (8..512 over caches read as bf16
     # hi + lo tiles: fp32, or fp16 under an fp32 q); checked before any HIP call
