@@ -1003,6 +1003,7 @@ extern "C" int64_t sa_flash_bwd_workspace_size(int B, int Hq, int Hkv, int T, in
     if (B < 0 || Hq <= 0 || Hkv <= 0 || T < 0 || D <= 0 || Hq % Hkv != 0 || window_size < 0) return -1;
     if (dtype != SA_BF16 && dtype != SA_F16) return 0;
     if (B == 0 || T == 0 || D > 512) return 0;
+    window_size = effective_window(window_size, T);
     if (D > 128) return flash_bwd_wide_workspace_size(B, Hq, Hkv, T, D, window_size);
     // room for the plans with and without groups (exact square roots have none, and then split more), and for
     // two splits in the smallest grids, also where none is chosen
@@ -1019,6 +1020,7 @@ extern "C" int sa_flash_bwd_plan(int B, int Hq, int Hkv, int T, int D, int windo
     if (!plan) return SA_ERR_NULL_POINTER;
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || Hq % Hkv != 0 || window_size < 0) return SA_ERR_BAD_SHAPE;
     if (D < 8 || D > 128 || D % 8 != 0) return SA_ERR_UNSUPPORTED;
+    window_size = effective_window(window_size, T);
     const BwdPlan p = choose_bwd_plan(B, Hkv, T, Hq / Hkv, window_size, D,
                                       splits_that_fit(B, Hkv, T, D, workspace_bytes), !exact_math);
     plan[0] = p.dq_groups;
@@ -1035,6 +1037,7 @@ extern "C" int sa_flash_bwd_ws(const void* q, const void* k, const void* v, cons
                                float scale, int window_size, int exact_math, int dtype, void* workspace,
                                int64_t workspace_bytes, sa_stream_t stream) {
     using namespace sa;
+    window_size = effective_window(window_size, T);
     if (dtype == SA_F32) {
         const int64_t* const all[8] = {q_strides,  k_strides,  v_strides,  o_strides,
                                        do_strides, dq_strides, dk_strides, dv_strides};

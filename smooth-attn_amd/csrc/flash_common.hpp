@@ -132,6 +132,11 @@ __device__ __forceinline__ void grouped_block(int id, int n_units, int n_sub, in
     }
 }
 
+// A window of the rows' length or more hides no key: no window (0) to the
+// choices and kernels, whose sums of a position and the window then stay in
+// 32 bits.
+inline int effective_window(int window_size, int T) { return window_size >= T && window_size > 0 ? 0 : window_size; }
+
 // squareplus(a)^2 with a = scale * s - 1/2 already folded in:
 //   squareplus(2 s scale - 1) = (2 s scale - 1 + sqrt((2 s scale - 1)^2 + 4)) / 2
 //                             = a + sqrt(a^2 + 1),   a = s scale - 1/2.

@@ -247,7 +247,7 @@ int fill_params(FlashParams& prm, const void* q, const void* k, const void* v, v
         prm.vs[i] = v_strides[i];
         prm.os[i] = o_strides[i];
     }
-    set_sizes(prm, B, Hq, Hkv, T, D, window_size);
+    set_sizes(prm, B, Hq, Hkv, T, D, effective_window(window_size, T));
     prm.scale = scale;
     return 0;
 }
@@ -264,7 +264,7 @@ extern "C" int sa_flash_fwd_key_split(int B, int Hq, int Hkv, int T, int D, int 
     if (D < 8 || D > 128 || D % 8 != 0) return SA_ERR_UNSUPPORTED;
     if (exact_math) return 1;
     FlashParams prm{};
-    set_sizes(prm, B, Hq, Hkv, T, D, window_size);
+    set_sizes(prm, B, Hq, Hkv, T, D, effective_window(window_size, T));
     prm.ks[2] = prm.vs[2] = kv_row_bytes;
     return key_split_for(prm, 1, 1);
 }
@@ -274,6 +274,7 @@ extern "C" int sa_flash_fwd(const void* q, const void* k, const void* v, void* o
                             const int64_t* v_strides, const int64_t* o_strides, float scale, int window_size,
                             int exact_math, int dtype, sa_stream_t stream) {
     using namespace sa;
+    window_size = effective_window(window_size, T);
     if (dtype == SA_F32)
         return flash_fwd_f32(q, k, v, o, row_sums, B, Hq, Hkv, T, D, q_strides, k_strides, v_strides, o_strides,
                              scale, window_size, exact_math, reinterpret_cast<hipStream_t>(stream));

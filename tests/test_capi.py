@@ -241,6 +241,23 @@ def test_attention_build_queries():
     assert query(1, 8, 1, 16384, 128, 0, 0, ws - 16, plan) == 0 and 1 <= plan[2] < n
 
 
+@pytest.mark.parametrize("window", [0, 1 << 30, (1 << 31) - 1])
+@pytest.mark.parametrize("heads,T,D", [((2, 32, 8), 3000, 128), ((1, 8, 2), 1025, 64), ((2, 16, 16), 2048, 256)])
+def test_windows_of_all_rows_choose_as_no_window(heads, T, D, window):
+    lib = _lib.load()
+    w = window or T  # the rows' length, and windows whose double is past 32 bits
+    assert lib.sa_flash_bwd_workspace_size(*heads, T, D, w, _lib.SA_BF16) == \
+        lib.sa_flash_bwd_workspace_size(*heads, T, D, 0, _lib.SA_BF16)
+    if D > 128:
+        return
+    assert lib.sa_flash_fwd_key_split(*heads, T, D, w, 0, 2 * D) == lib.sa_flash_fwd_key_split(*heads, T, D, 0, 0, 2 * D)
+    for exact in (0, 1):
+        a, b = (ctypes.c_int * 3)(), (ctypes.c_int * 3)()
+        assert lib.sa_flash_bwd_plan(*heads, T, D, w, exact, 1 << 40, a) == 0
+        assert lib.sa_flash_bwd_plan(*heads, T, D, 0, exact, 1 << 40, b) == 0
+        assert list(a) == list(b)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,T,D,window", [
     (4, 32, 8, 512, 64, 128), (1, 32, 32, 1024, 64, 0), (1, 32, 8, 2048, 128, 0), (1, 8, 8, 4096, 128, 0),
     (2, 16, 16, 1024, 32, 0), (8, 32, 8, 300, 64, 0), (2, 12, 12, 1280, 128, 0), (1, 4, 4, 314, 96, 0)])

@@ -213,3 +213,19 @@ def test_full_size_head_dim_256_sampled():
     refs = eager.flash_attention_bwd(*(t[sl].cpu().double() for t in (q, k, v, o, do)))
     for got, want in zip((dq, dk, dv), refs):
         assert rel_err(got[sl], want) <= TOL
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256), (torch.float32, 64)])
+def test_windows_of_all_rows_are_no_window(dtype, D):
+    # a window of T or more keys hides none, up to the largest int: position
+    # plus window must not leave 32 bits
+    q, k, v, do = (torch.randn(1, h, 333, D, generator=_g(h)).to(dtype).to(DEV) for h in (4, 2, 2, 4))
+
+    def step(window):
+        a = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = smooth_attn.sp2norm_flash_attention(*a, window_size=window)
+        return (o, *torch.autograd.grad(o, a, do))
+    want = step(0)
+    for window in (333, 334, 1 << 30, (1 << 31) - 1):
+        for x, y in zip(step(window), want):
+            assert torch.equal(x, y), window
