@@ -1,12 +1,10 @@
-// Host-side pieces of the dK/dV query-range split: the makespan estimate by
-// which the backward for head dims 136..512 chooses its split count, and a
-// small cache of choices shared with the backward for head dims up to 128.
+// Host-side piece of the dK/dV query-range split: the makespan estimate by
+// which the backward for head dims 136..512 chooses its split count.
 #pragma once
 
 #include <algorithm>
 #include <cstdint>
 #include <functional>
-#include <mutex>
 #include <vector>
 
 namespace sa {
@@ -38,37 +36,5 @@ double dkdv_split_makespan(int nkb, int units, int n_split, int slots, double se
     }
     return *std::max_element(heap.begin(), heap.end()) + 0.2 * longest;
 }
-
-// The split counts of the last 16 shapes asked for (the estimate costs up to
-// ~0.1 ms of host time, and a training step asks for the same shapes again).
-class SplitCountCache {
-  public:
-    template <typename Compute>
-    int get(const int (&key)[6], Compute compute) {
-        {
-            std::lock_guard<std::mutex> lock(mu_);
-            for (int i = 0; i < n_cached_; ++i)
-                if (std::equal(key, key + 6, cache_[i].key)) return cache_[i].n_split;
-        }
-        const int n = compute();
-        std::lock_guard<std::mutex> lock(mu_);
-        Entry& e = cache_[next_];
-        std::copy(key, key + 6, e.key);
-        e.n_split = n;
-        next_ = (next_ + 1) % kEntries;
-        n_cached_ = std::min(n_cached_ + 1, kEntries);
-        return n;
-    }
-
-  private:
-    static constexpr int kEntries = 16;
-    struct Entry {
-        int key[6];
-        int n_split;
-    };
-    std::mutex mu_;
-    Entry cache_[kEntries];
-    int n_cached_ = 0, next_ = 0;
-};
 
 }  // namespace sa

@@ -36,7 +36,8 @@
 #include "flash_tiles.hpp"
 #include "flash_f32.hpp"
 #include "flash_wide.hpp"
-#include "dkdv_split.hpp"
+#include "block_order.hpp"
+#include "choice_cache.hpp"
 
 #include <algorithm>
 
@@ -986,7 +987,7 @@ int splits_that_fit(int B, int Hkv, int T, int dr, int64_t workspace_bytes) {
 BwdPlan choose_bwd_plan(int B, int Hkv, int T, int G, int W, int dr, int max_split, bool groups) {
     const int64_t blocks = static_cast<int64_t>((T + kBwdBK - 1) / kBwdBK) * B * Hkv;
     if (blocks >= 8 * kBwdXcdSlots * 8 || blocks == 0) return BwdPlan{};  // full grids
-    static SplitCountCache cache;  // (a plan is kept as one number)
+    static ChoiceCache cache;  // (a plan is kept as one number)
     const int key[6] = {B, Hkv, T, G, W, (bwd_kernel_d(dr) << 8) | (max_split << 1) | (groups ? 1 : 0)};
     const int code = cache.get(key, [&] {
         const BwdPlan p = choose_bwd_plan_uncached(B, Hkv, T, G, W, dr, max_split, groups);

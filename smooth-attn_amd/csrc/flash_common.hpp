@@ -84,30 +84,8 @@ __device__ __forceinline__ V lds_read_tr16_pair(const void* p0, const void* p1) 
 // and the group's heavy steps still start early.  Otherwise step-major over
 // all (unit, sub).
 //
-// `uneven` (steps differ in work): where a group's blocks are no multiple of
-// xcd_slots, the next group's heavy steps start late and the last group's end
-// late, up to half again the balanced time in grids of a few rounds.  Up to
-// kOneGroupRounds blocks per slot an XCD then takes all its units as one
-// group, heavy steps first throughout (as groups -> as one; bf16, D = 128,
-// forward / backward us: [1,32,3000] 126 / 397 -> 102 / 341, [2,32,1536] 71 /
-// 227 -> 58 / 193, [4,32,3000], 6 rounds, 400 / 1236 -> 374 / 1152).  Longer
-// grids lose more L2 hits than they gain ([4,32,5000], 10 rounds, 931 / 3022
-// -> 934 / 3080), and so do equal steps ([2,32/8,3000] window 1024 forward 122
-// -> 125).
-constexpr int kOneGroupRounds = 8;
-__host__ __device__ __forceinline__ int units_per_group(int n_units, int n_sub, int n_steps, int xcd_slots,
-                                                        bool uneven) {
-    // blocks of a unit (none in an empty call, which launches nothing), units of an XCD
-    const int per = n_sub * n_steps > 0 ? n_sub * n_steps : 1, units = n_units >> 3;
-    int gu = (xcd_slots + per - 1) / per;
-    if (gu < 1) gu = 1;
-    if (gu > units) gu = units;
-    if (uneven && units * per <= kOneGroupRounds * xcd_slots && gu * per % xcd_slots != 0) gu = units;
-    return gu;
-}
-
-// gu: units_per_group of the same grid (read only where n_units is a multiple
-// of 8, and then at least 1).
+// gu: units per group, from block_order.hpp (read only where n_units is a
+// multiple of 8, and then at least 1).
 __device__ __forceinline__ void grouped_block(int id, int n_units, int n_sub, int n_steps, int gu, int& step,
                                               int& unit, int& sub) {
     if ((n_units & 7) == 0) {

@@ -160,8 +160,9 @@ int key_split_for(const FlashParams& p, int qk_bytes, int v_bytes) {
 }
 
 template <typename T, int D, bool QK8, bool V8>
-int launch_flash(const FlashParams& prm, int exact, hipStream_t st) {
+int launch_flash(FlashParams prm, int exact, hipStream_t st) {
     if (exact) {
+        set_grid(prm, Split<1>::BQ, Split<1>::BKV);
         const dim3 grid(static_cast<unsigned>(prm.nqb) * prm.B * prm.Hq);
         flash_fwd_kernel<T, D, QK8, V8, true, false><<<grid, dim3(kThreads), 0, st>>>(prm);
         return status_from_launch();
@@ -220,7 +221,7 @@ void set_sizes(FlashParams& prm, int B, int Hq, int Hkv, int T, int D, int windo
     prm.G = Hq / Hkv;
     prm.window = window_size;
     prm.dr = D;
-    set_grid(prm, Split<1>::BQ);
+    prm.nqb = (T + Split<1>::BQ - 1) / Split<1>::BQ;
 }
 
 int fill_params(FlashParams& prm, const void* q, const void* k, const void* v, void* o, float* row_sums, int B,

@@ -26,8 +26,11 @@
 // Block order: see block_coords (XCD-aware, heaviest query blocks first).
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
+#include "block_order.hpp"
+#include "choice_cache.hpp"
 #include "flash_common.hpp"
 #include "flash_tiles.hpp"
 
@@ -147,17 +150,31 @@ __device__ __forceinline__ u32x4 tile_load16(const T* p) {
 // one block per CU, so an XCD runs 32 at once.
 constexpr int kBlocksPerXcd = 32;
 
-// Query blocks of bq rows and their order.  The group size is worked out here,
-// once: in the kernel its divisions stood before every block's first load
-// (forward, means of two runs: [2,32/8,1152,96] 35.8 -> 35.3 us,
-// [1,32/8,512,128] 11.6 -> 11.4, [8,32,878,80] 86.3 -> 85.9).
-inline void set_grid(FlashParams& p, int bq) {
+// Query blocks of bq rows, their order and the key tiles of bkv keys.  The
+// group size is worked out here, once: in the kernel its divisions stood
+// before every block's first load (forward, means of two runs: [2,32/8,1152,96]
+// 35.8 -> 35.3 us, [1,32/8,512,128] 11.6 -> 11.4, [8,32,878,80] 86.3 -> 85.9).
+inline void set_grid(FlashParams& p, int bq, int bkv) {
     p.nqb = (p.T + bq - 1) / bq;
     // (under a window of up to half the rows most query blocks walk equally
     // many tiles; and groups of one KV head that fill the XCD by themselves
     // are balanced within 5%, where the L2 hits count more)
     const bool uneven = (p.window <= 0 || 2 * p.window > p.T) && p.G * p.nqb <= kBlocksPerXcd;
-    p.group_units = units_per_group(p.B * p.Hkv, p.G, p.nqb, kBlocksPerXcd, uneven);
+    const int units = p.B * p.Hkv, groups = units_per_group(units, p.G, p.nqb, kBlocksPerXcd, false);
+    p.group_units = units_per_group(units, p.G, p.nqb, kBlocksPerXcd, uneven);
+    if (p.group_units == groups || p.dr <= 64) return;  // (D <= 64: see units_per_group)
+    static ChoiceCache cache;
+    const int key[6] = {units, p.G, p.T, p.window, bq, bkv};
+    p.group_units = cache.get(key, [&] {
+        const int n_kv = (p.T + bkv - 1) / bkv;
+        const double setup = bq == Split<1>::BQ ? 1.4 : 6.0;  // of a block, in key tiles
+        const auto cost = [&](int step) {
+            const int q0 = (p.nqb - 1 - step) * bq;
+            const int first = p.window > 0 ? std::max(0, q0 - p.window + 1) / bkv : 0;
+            return std::min((q0 + bq + bkv - 1) / bkv, n_kv) - first + setup;
+        };
+        return order_gain(units, p.G, p.nqb, groups, kBlocksPerXcd, cost) ? units >> 3 : groups;
+    });
 }
 
 __device__ __forceinline__ void block_coords(const FlashParams& p, int& qb, int& b, int& hq) {
@@ -611,10 +628,15 @@ __global__ __launch_bounds__(kThreads, KS == 2 && D == 64 ? 4 : 1) void flash_fw
     // or NaN of V (times a weight of 0) then reaches the rows that it reaches
     // under every key split.
     const int wf = wq0[0], wl = wq0[kQT - 1] + 31;
-    const int part0 = KS == 4 ? (grp >> 1) * 64 : 0;  // first of those keys in the tile
-    int t_first = kv_begin;
-    if (W > 0 && wf - W + 1 > 0) t_first = max(t_first, (wf - W + 1 + kBKV - 64 - part0) / kBKV);
-    const int t_last = wf < T_ ? min((wl - part0) >> (KS == 4 ? 7 : 6), kv_end - 1) : t_first - 1;
+    int t_first = kv_begin, t_last = t_first - 1;
+    if constexpr (KS == 4) {
+        const int part0 = (grp >> 1) * 64;  // first of those keys in the tile
+        if (W > 0 && wf - W + 1 > 0) t_first = max(t_first, (wf - W + 1 + kBKV - 64 - part0) / kBKV);
+        t_last = wf < T_ ? min((wl - part0) >> 7, kv_end - 1) : t_first - 1;
+    } else {
+        if (W > 0 && wf - W + 1 > 0) t_first = max(t_first, (wf - W + 1) / kBKV);
+        t_last = wf < T_ ? min(wl / kBKV, kv_end - 1) : t_first - 1;
+    }
     int ja = t_first;
     if (W > 0 && wl - W >= 0) ja = max(ja, (wl - W) / kBKV + 1);
     const int jb = (wf + 1) / kBKV;
@@ -778,7 +800,7 @@ bool fold_scale_ok(float scale) {
 // One launch of the kernel with key split KS (not for exact math).
 template <typename T, int D, bool QK8, bool V8, bool ROPE, int KS>
 int launch_flash_split(FlashParams prm, hipStream_t st) {
-    set_grid(prm, Split<KS>::BQ);
+    set_grid(prm, Split<KS>::BQ, Split<KS>::BKV);
     const dim3 grid(static_cast<unsigned>(prm.nqb) * prm.B * prm.Hq);
     if constexpr (kCanFold<T, QK8, D>) {
         if (fold_scale_ok<QK8>(prm.scale)) {

@@ -38,6 +38,8 @@
 
 #include "flash_tiles.hpp"
 #include "flash_wide.hpp"
+#include "block_order.hpp"
+#include "choice_cache.hpp"
 #include "dkdv_split.hpp"
 
 namespace sa {
@@ -59,6 +61,7 @@ struct WideParams {
     float* delta;  // [B, Hq, T]
     int64_t qs[4], ks[4], vs[4], os[4], dos[4], dqs[4], dks[4], dvs[4];
     int B, Hq, Hkv, T, G, window;
+    int group_units;  // units_per_group of the forward's or the dQ kernel's grid
     int dr;  // head dim of the tensors (<= D, a multiple of 8; columns past it read as zero, are not stored)
     float scale;
     int n_split;  // dK/dV: query-range splits of every key block (1: none)
@@ -212,8 +215,7 @@ __global__ __launch_bounds__(64 * WideCfg<D>::NW) void flash_fwd_wide_kernel(Wid
     const int T_ = p.T;
     const int nqb = (T_ + kFRows - 1) / kFRows;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, units_per_group(p.B * p.Hkv, p.G, nqb, 32, true), step, unit,
-                  sub);  // heaviest query blocks first
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, p.group_units, step, unit, sub);  // heaviest query blocks first
     const int qb = nqb - 1 - step;
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
@@ -433,8 +435,7 @@ __global__ __launch_bounds__(64 * WideCfg<D>::NW) void flash_bwd_dq_wide_kernel(
     const int T_ = p.T;
     const int nqb = (T_ + kFRows - 1) / kFRows;
     int step, unit, sub;
-    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, units_per_group(p.B * p.Hkv, p.G, nqb, 32, false), step, unit,
-                  sub);
+    grouped_block(blockIdx.x, p.B * p.Hkv, p.G, nqb, p.group_units, step, unit, sub);
     const int qb = nqb - 1 - step;
     const int b = unit / p.Hkv;
     const int hk = unit - b * p.Hkv;
@@ -903,11 +904,15 @@ int check_wide(int B, int Hq, int Hkv, int T, int D, int window_size, int dtype)
     return 0;
 }
 
+constexpr int kWideBlocksPerXcd = 32;  // one block per CU
+
 template <typename T, int D>
-int launch_fwd_wide(const WideParams<T>& prm, int exact, hipStream_t st) {
+int launch_fwd_wide(WideParams<T> prm, int exact, hipStream_t st) {
     constexpr int kFW = WideCfg<D>::NW, kFRows = WideCfg<D>::ROWS;
-    const int64_t nblk = static_cast<int64_t>((prm.T + kFRows - 1) / kFRows) * prm.B * prm.Hq;
+    const int nqb = (prm.T + kFRows - 1) / kFRows;
+    const int64_t nblk = static_cast<int64_t>(nqb) * prm.B * prm.Hq;
     if (nblk * 64 * kFW >= (int64_t(1) << 32)) return SA_ERR_BAD_SHAPE;
+    prm.group_units = units_per_group(prm.B * prm.Hkv, prm.G, nqb, kWideBlocksPerXcd, true);
     const dim3 grid(static_cast<unsigned>(nblk));
     if (exact) {
         flash_fwd_wide_kernel<T, D, true, false><<<grid, 64 * kFW, 0, st>>>(prm);
@@ -939,13 +944,15 @@ void launch_bwd_wide_kernels(const WideParams<T>& prm, dim3 gq, dim3 gk, hipStre
 }
 
 template <typename T, int D, bool PART>
-int launch_bwd_wide_part(const WideParams<T>& prm, int exact, hipStream_t st) {
+int launch_bwd_wide_part(WideParams<T> prm, int exact, hipStream_t st) {
     constexpr int kFW = WideCfg<D>::NW, kFRows = WideCfg<D>::ROWS;
-    const int64_t nq = static_cast<int64_t>((prm.T + kFRows - 1) / kFRows) * prm.B * prm.Hq;
+    const int nqb = (prm.T + kFRows - 1) / kFRows;
+    const int64_t nq = static_cast<int64_t>(nqb) * prm.B * prm.Hq;
     if (nq * 64 * kFW >= (int64_t(1) << 32)) return SA_ERR_BAD_SHAPE;  // dQ blocks of kFW waves
     const int64_t nk = nq / prm.G * prm.n_split;
     if (nk * 64 * kFW >= (int64_t(1) << 32)) return SA_ERR_BAD_SHAPE;
     const dim3 gq(static_cast<unsigned>(nq)), gk(static_cast<unsigned>(nk));
+    prm.group_units = units_per_group(prm.B * prm.Hkv, prm.G, nqb, kWideBlocksPerXcd, false);
     if (exact) launch_bwd_wide_kernels<T, D, true, PART>(prm, gq, gk, st);
     else launch_bwd_wide_kernels<T, D, false, PART>(prm, gq, gk, st);
     return status_from_launch();
@@ -1043,7 +1050,7 @@ int wide_split_count(int B, int Hkv, int T, int G, int W, int dr) {
     const int R = dr <= 256 ? WideCfg<256>::ROWS : WideCfg<512>::ROWS;  // key rows per block
     const int64_t blocks = static_cast<int64_t>((T + R - 1) / R) * B * Hkv;
     if (blocks >= 8 * 32 * 8 || blocks == 0) return 1;
-    static SplitCountCache cache;
+    static ChoiceCache cache;
     const int key[6] = {B, Hkv, T, G, W, wide_kernel_d(dr)};
     return cache.get(key, [&] {
         return dr <= 256 ? wide_split_count_uncached<256>(B, Hkv, T, G, W)
