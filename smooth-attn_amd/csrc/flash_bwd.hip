@@ -873,14 +873,15 @@ int dkdv_iterations(int kb, int T, int G, int W) {
 //    summed by one more kernel.
 // Each candidate is estimated as the longer of the longest block and all
 // work shared out evenly, plus a part of the other (the ragged end), plus the
-// partials' traffic; constants in us, fitted to 430 measured shapes (bf16,
-// D = 64 to 128, T = 256 .. 8192, up to 1100 blocks of 256 rows, GQA 1 to 8,
-// windows of none to half), on which the choice averages 0.3% over the
-// fastest candidate and is at worst 7% over it.  dQ + dK/dV, one group and
-// the S of an earlier rule -> two groups or another S: [4,12,1024,64] 68 ->
-// 55 us, [1,32,1024,128] 91 -> 73, [1,32,2048,128] 195 -> 162,
-// [2,32/8,3000,128] window 1024 (S = 4 -> 1) 419 -> 382, [1,32/8,2048,128] 199
-// -> 168; full grids keep one group.
+// partials' traffic; constants in us, fitted to the 463 measured shapes of
+// profiles/attention_bwd_plan_us.csv (bf16, T = 256 .. 8192, up to 1100 blocks
+// of 256 rows, GQA 1 to 8, windows of none to most), on which the chosen dK/dV
+// plan averages 0.3% over the fastest and is at worst 5% over it, dQ's groups
+// 0.2% and 5%, exact square roots' splits (one group always) 0.6% and 11%.
+// dQ + dK/dV, one group and the S of an earlier rule -> two groups or another
+// S: [4,12,1024,64] 68 -> 55 us, [1,32,1024,128] 91 -> 73, [1,32,2048,128] 195
+// -> 162, [2,32/8,3000,128] window 1024 (S = 4 -> 1) 419 -> 382,
+// [1,32/8,2048,128] 199 -> 168; full grids keep one group.
 struct BwdCosts {
     // by groups - 1: setup and tile of the longest block, the same of a block in a full grid (per CU);
     // *_alone: a tile of a one-group block that has its CU to itself
@@ -889,14 +890,10 @@ struct BwdCosts {
     double part_tb_s, part_setup;
     double exact_iter;  // an iteration with exact square roots, times the above
 };
-// Exact square roots (one group always), fitted to 80 shapes of the same
-// ranges: the choice averages 0.6% over the fastest S, without the factors
-// 1.8% and at worst 20% ([2,12,1280,128]: S = 1 / 2 / 4 151 / 135 / 143 us).
-constexpr double kExactPart = 0.7;  // their part of part_setup
 constexpr BwdCosts kBwdCosts128 = {{3.5, 10.7}, 2.14, {2.43, 0.89}, {6.8, 5.7}, {0.43, 1.74}, 0.41,
-                                   6.4, 2.79, {3.33, 2.72}, {7.0, 9.9}, {1.85, 2.53}, 0.05, 8.0, 14.3, 1.6};
+                                   7.2, 2.79, {3.3, 2.72}, {7.5, 9.9}, {2.0, 2.57}, 0.066, 8.2, 9.2, 1.7};
 constexpr BwdCosts kBwdCosts64 = {{3.7, 10.5}, 2.02, {1.88, 0.96}, {5.7, 8.0}, {1.06, 1.63}, 0.09,
-                                  12.5, 2.59, {2.59, 1.54}, {3.3, 10.2}, {1.59, 2.42}, 0.38, 5.0, 4.2, 1.3};
+                                  18.1, 2.59, {2.41, 1.54}, {4.3, 12.5}, {1.59, 1.96}, 0.50, 7.0, 5.3, 1.2};
 
 struct BwdPlan {
     int dq_groups = 1, kv_groups = 1, n_split = 1;
@@ -915,7 +912,6 @@ BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, in
         c.kv_alone *= c.exact_iter;
         c.kv_iter[0] *= c.exact_iter;
         c.kv_share[0] *= c.exact_iter;
-        c.part_setup *= kExactPart;
     }
     const int nkb = (T + kBwdBK - 1) / kBwdBK, nqb = (T + kBwdBQ - 1) / kBwdBQ;
     const int n_kv = (T + kBwdKT - 1) / kBwdKT;
@@ -938,12 +934,6 @@ BwdPlan choose_bwd_plan_uncached(int B, int Hkv, int T, int G, int W, int dr, in
     const auto tile_time = [](double alone, double shared, double blocks) {
         return alone + (shared - alone) * std::min(1.0, std::max(0.0, blocks / kCus - 1.0));
     };
-    // Under a window of up to half the rows the blocks are nearly equal; where
-    // all run at once on most of the slots (D = 128: two blocks per CU) neither
-    // shortens the whole ([2,32/8,3000] window 1024: S = 1 / 2 / 4, two groups
-    // 382 / 411 / 419, 442 us).
-    if (W > 0 && 2 * W <= T && bwd_kernel_d(dr) == 128 && nkb * kv_heads > 1.25 * kCus && nkb * kv_heads <= 2 * kCus)
-        max_split = 0;
     BwdPlan best;
     double dq_t = 0.0, kv_t = 0.0;
     for (int g = 0; g < (groups ? 2 : 1); ++g) {

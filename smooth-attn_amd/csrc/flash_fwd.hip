@@ -133,9 +133,12 @@ double forward_estimate(const FlashParams& p, const SplitCosts& c, double ragged
 // that leave CUs idle or waiting for the longest block, but costs a merge and
 // more barriers per MFMA, so full grids keep KS = 1 at D = 128; at D = 64 two
 // KS = 2 blocks fit a CU (under 128 registers) and it wins over most sizes.
-// The constants (us) are fitted to 430 measured shapes (bf16, T = 256 ..
-// 8192, up to 1100 blocks of 256 rows, GQA 1 to 8, windows of none to half),
-// on which the choice averages 0.3% over the fastest KS.  KS = 1 / 2 / 4 in us,
+// The constants (us) are fitted to measured shapes of D = 64 to 128 (bf16, T =
+// 256 .. 8192, up to 1100 blocks of 256 rows, GQA 1 to 8, windows of none to
+// most).  On the 811 of profiles/attention_fwd_key_split_us.csv the choice
+// averages 1.1% over the fastest KS at D = 72 to 128, 0.5% at D = 40 to 64 and
+// 6% at D = 32, which shares their constants; against KS = 1 throughout it takes
+// 0.84, 0.80 and 0.79 of the time, at worst 1.18.  KS = 1 / 2 / 4 in us,
 // D = 128: [1,32/8,512] 18.7 / 15.3 / 13.1, [1,32/8,1024] 31.4 / 23.4 / 26.2,
 // [1,32/8,2048] 58.0 / 52.4 / 69.9, [1,8,2048] 54.3 / 35.5 / 25.6,
 // [2,32/8,1024] 34.0 / 35.3 / 49.4; D = 64: [1,32/8,5760] 207 / 179 / 251.

@@ -40,14 +40,15 @@ def grads64(q, k, v, o, do, window):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,Hq,Hkv,T,D,window", [
-    (2, 8, 8, 512, 128, 0), (2, 8, 8, 513, 64, 0), (1, 8, 8, 575, 32, 0), (2, 4, 4, 640, 96, 0), (1, 8, 8, 700, 40, 0),
-    (1, 16, 4, 577, 64, 0), (1, 8, 2, 1025, 128, 0), (1, 8, 8, 900, 128, 130), (1, 8, 2, 800, 64, 65),
-    (1, 4, 4, 1100, 128, 1), (1, 16, 2, 600, 80, 333)])
-def test_groups_match_float64(dtype, B, Hq, Hkv, T, D, window):
-    # (a window of 1 leaves the dQ blocks, and at D = 128 the dK/dV blocks, nothing to share)
-    dq_groups, kv_groups, _ = plan(B, Hq, Hkv, T, D, window)
-    assert (kv_groups == 2) == (window != 1) and (dq_groups == 2 or 0 < window <= 130)
+@pytest.mark.parametrize("B,Hq,Hkv,T,D,window,groups", [
+    (2, 8, 8, 512, 128, 0, (2, 2)), (2, 8, 8, 513, 64, 0, (2, 2)), (1, 8, 8, 575, 32, 0, (2, 2)),
+    (2, 4, 4, 640, 96, 0, (2, 2)), (1, 8, 8, 700, 40, 0, (2, 1)), (1, 8, 8, 575, 40, 0, (2, 2)),
+    (1, 16, 4, 577, 64, 0, (2, 2)), (1, 8, 2, 1025, 128, 0, (2, 2)), (1, 8, 8, 900, 128, 130, (1, 2)),
+    (1, 8, 8, 900, 128, 400, (2, 2)), (1, 8, 2, 800, 64, 65, (1, 2)), (1, 4, 4, 1100, 128, 1, (1, 1)),
+    (1, 16, 2, 600, 80, 333, (2, 2))])
+def test_groups_match_float64(dtype, B, Hq, Hkv, T, D, window, groups):
+    # groups of the dQ and the dK/dV blocks: short windows leave them little to share
+    assert plan(B, Hq, Hkv, T, D, window)[:2] == groups
     g = torch.Generator().manual_seed(T + D)
     mk = lambda H: torch.randn(B, T, H, D, generator=g).to(dtype).transpose(1, 2)  # rows of all heads side by side
     q, k, v, do = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
@@ -67,9 +68,9 @@ def test_groups_match_float64(dtype, B, Hq, Hkv, T, D, window):
 
 def test_exact_square_roots_keep_one_group():
     # (no two-group build): same gradients as the fast build within rounding
-    assert plan(1, 8, 8, 700, 64, 0)[:2] == (2, 2) and plan(1, 8, 8, 700, 64, 0, 1)[:2] == (1, 1)
+    assert plan(1, 8, 8, 513, 64, 0)[:2] == (2, 2) and plan(1, 8, 8, 513, 64, 0, 1)[:2] == (1, 1)
     g = torch.Generator().manual_seed(1)
-    q, k, v, do = (torch.randn(1, 8, 700, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
+    q, k, v, do = (torch.randn(1, 8, 513, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
     o, rs = kernels._sp2norm_flash_fwd(q, k, v, 0.125, 1, 0)
     a = kernels._sp2norm_flash_bwd(q, k, v, o, do, rs, 0.125, 1, 0)
     b = kernels._sp2norm_flash_bwd(q, k, v, o, do, rs, 0.125, 1, 0, use_fast_sqrt=False)
