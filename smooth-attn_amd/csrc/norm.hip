@@ -38,11 +38,12 @@ constexpr int fwd_waves() {
     // raw words + fp32 weights
     return waves_for_live(NCH * 4 + NCH * (16 / static_cast<int>(sizeof(T))));
 }
-template <typename T, typename TG, int NCH>
+template <typename T, typename TG, int NCH, bool ANY>
 constexpr int bwd_waves() {
     constexpr int vec = 16 / static_cast<int>(sizeof(T));
-    // dy words + one fp32 array + (on average) half of the x words
-    return waves_for_live(NCH * 2 + NCH * vec * static_cast<int>(sizeof(TG)) / 4 + NCH * vec);
+    // dy words + one fp32 array + (on average) half of the x words; ANY keeps
+    // each chunk's first column and its lane's place in it
+    return waves_for_live(NCH * 2 + NCH * vec * static_cast<int>(sizeof(TG)) / 4 + NCH * vec + (ANY ? 2 * NCH : 0));
 }
 
 template <int POWER>
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fwd_waves<T
 }
 
 template <typename T, typename TG, int NCH, int POWER, bool ANY = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T, TG, NCH>(), 8))) void norm_bwd_vec(const T* __restrict__ x, const TG* __restrict__ dy,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_waves<T, TG, NCH, ANY>(), 8))) void norm_bwd_vec(const T* __restrict__ x, const TG* __restrict__ dy,
                                                     T* __restrict__ dx, int64_t n_rows, int n_cols,
                                                     int64_t xs, int64_t gs, int64_t dxs, int causal,
                                                     float alpha, float neg_alpha_theta,
