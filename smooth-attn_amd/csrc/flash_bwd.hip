@@ -464,9 +464,14 @@ __global__ __launch_bounds__(kBwdThreads * KS, KS == 1 ? kBwdDkdvMinBlocks : 1) 
     // 32-query half.  The 128 accumulators plus all of K and V leave no room
     // under 256 registers, and a compiler spill instead reloads from scratch
     // inside the tile loop, where the wait for it (memory loads complete in
-    // order) also waits for the next tile's DMA.  (With fast square roots
-    // this leaves no spill; the exact-sqrt build keeps 12 bytes.)
-    constexpr int NXK = D == 128 ? (KS == 2 ? 5 : kDkdvLdsK) : 0, NXV = D == 128 ? kDkdvLdsV : 0;
+    // order) also waits for the next tile's DMA.  (At dr = 128 the one-group
+    // builds keep 16 bytes spilled, reloaded after the loop, and with exact
+    // square roots 20, of which 4 in it.  Two groups: 5 K chunks alone spill 20
+    // bytes with reloads in the loop, with a V chunk none, [1,32,1024,128]
+    // backward 73.5 -> 71.2 us, [1,8,4096,128] 199.5 -> 196.4; below dr = 128 no
+    // chunk of V is needed and it costs, [1,32,1500,96] 92.5 -> 93.7.)
+    constexpr int NXK = D == 128 ? (KS == 2 ? 5 : kDkdvLdsK) : 0;
+    constexpr int NXV = D == 128 ? (KS == 2 && !PART ? 1 : kDkdvLdsV) : 0;
     __shared__ __attribute__((aligned(16))) u32x4 kvx[NXK + NXV > 0 ? NXK + NXV : 1][4 * KS][64];  // [K chunks, V chunks][wave][lane]
     constexpr bool HALFX = D == 128;
     __shared__ __attribute__((aligned(16))) uint2 kvh[HALFX ? 4 * KS : 1][64];  // [wave][lane]: low 8 bytes of K chunk NXK
