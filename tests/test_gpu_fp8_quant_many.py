@@ -63,3 +63,33 @@ def test_infinite_scale():
     for x8, scale in many:
         assert float(scale) == float("inf")
         assert torch.equal(x8.view(torch.uint8), wide[0].view(torch.uint8))
+
+
+def _one_word(x, dirty):
+    """sa_fp8_quantize: one word of workspace, whatever it holds."""
+    from smooth_attn import _lib
+
+    lib = _lib.load()
+    x8 = torch.full((max(x.numel(), 1),), 0x55, dtype=torch.uint8, device=DEV)
+    ws = torch.tensor([dirty], dtype=torch.int32, device=DEV)
+    scale = torch.zeros(1, dtype=torch.float32, device=DEV)
+    st = lib.sa_fp8_quantize(x.data_ptr(), x8.data_ptr(), x.numel(), kernels._DTYPE_CODE[x.dtype], ws.data_ptr(),
+                             scale.data_ptr(), kernels._stream(x8))
+    assert st == 0
+    return x8, scale
+
+
+# a lone element, remainders, one block, the most blocks that meet in the word
+# (256, one per CU) and several loads of each; an address between 16-byte ones;
+# nothing at all; a workspace that holds zero, a large float's bits, NaN bits
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,offset", [(0, 0), (1, 0), (7, 0), (8192, 0), (8193, 1), (70_001, 1), (1 << 21, 0), (9_000_011, 0)])
+def test_one_word_workspace_matches_many(dtype, n, offset):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = (torch.randn(n + offset, generator=g, device=DEV) * 3).to(dtype)[offset:]
+    (want8, want), = kernels._quantize_many_to_fp8_device(x)
+    for dirty in (0, 0x7F000000, -1):
+        x8, scale = _one_word(x, dirty)
+        assert torch.equal(scale, want.reshape(1))
+        assert torch.equal(x8[:n], want8.view(torch.uint8).reshape(-1))
+        assert n > 0 or int(x8[0]) == 0x55  # nothing written
