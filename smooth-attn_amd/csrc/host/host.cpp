@@ -240,19 +240,21 @@ struct CausalNorm : public torch::autograd::Function<CausalNorm> {
                           "the saved x must have grad_output's shape and a dtype of the fused kernels");
         const int64_t cols = saved.size(-1);
         // (unpack hooks may hand back another layout or type than forward saved)
-        Tensor x = saved.reshape({-1, cols});
-        if (x.stride(1) != 1 || x.stride(0) < cols) x = x.contiguous();
+        const bool as_saved = saved.is_contiguous();
+        Tensor x = as_saved ? saved : saved.reshape({-1, cols});
+        if (!as_saved && (x.stride(1) != 1 || x.stride(0) < cols)) x = x.contiguous();
         if (g.scalar_type() != at::kFloat && g.scalar_type() != x.scalar_type()) g = g.to(at::kFloat);
         g = g.contiguous();
         Tensor dx = at::empty_like(x);
         const c10::DeviceGuard guard(x.device());
-        check(abi.norm_bwd(x.data_ptr(), g.data_ptr(), dx.data_ptr(), x.size(0), cols, x.stride(0), cols, dx.stride(0),
+        check(abi.norm_bwd(x.data_ptr(), g.data_ptr(), dx.data_ptr(), x.numel() / cols, cols, x.stride(-2), cols,
+                           dx.stride(-2),
                            code_of(x.scalar_type()), code_of(g.scalar_type()), 1,
                            static_cast<float>(ctx->saved_data["alpha"].toDouble()),
                            static_cast<float>(ctx->saved_data["theta"].toDouble()),
                            static_cast<int>(ctx->saved_data["power"].toInt()), stream_of(x)),
               "sa_norm_bwd");
-        return {dx.view(saved.sizes()), Tensor(), Tensor(), Tensor()};
+        return {as_saved ? dx : dx.view(saved.sizes()), Tensor(), Tensor(), Tensor()};
     }
 };
 
