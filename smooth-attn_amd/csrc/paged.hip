@@ -83,53 +83,61 @@ __device__ __forceinline__ int wave_prefix(int v) {
     return v;
 }
 
-// The plan as one wave sees it.  Up to kRegSeqs sequences every wave works
-// the plan out for itself, lane b holding sequence b: one load of the context
-// lengths and a wave scan, where the plan kernel costs a launch and the
+// The plan as one wave sees it.  Up to kRegSeqs sequences (REGS) every wave
+// works the plan out for itself, lane b holding sequence b: one load of the
+// context lengths and a wave scan, where the plan kernel costs a launch and the
 // waves a chain of dependent loads of what it wrote.  With the merge below, 8
 // sequences of 64 to 2048 tokens (Hq 32 / Hkv 8, D 128) 26.8 -> 17.8 us, one
 // of 16384 24.1 -> 13.9 us, 64 of 512 to 16384 tokens 1% faster; the same
 // bits.  Larger batches (one lane would hold several sequences) read the plan
-// kernel's, 2% of the time at 100 sequences.
+// kernel's, in builds of their own (both ways in one cost either about half a
+// microsecond a call).
 constexpr int kRegSeqs = 64;
+template <bool REGS>
 struct WavePlan {
     const PagedParams& p;
-    bool regs;      // wave-uniform
     int ctx, last;  // lane b: context length of sequence b, plan[b + 1]
     int Tt, Ne;
-    __device__ __forceinline__ explicit WavePlan(const PagedParams& prm) : p(prm), regs(prm.B <= kRegSeqs) {
-        if (regs) {
+    __device__ __forceinline__ explicit WavePlan(const PagedParams& prm) : p(prm) {
+        if constexpr (REGS) {
             const int b = threadIdx.x & 63;
             ctx = b < p.B ? ctx_of(p, b) : 0;
             last = wave_prefix(tiles_of(p, ctx));
             Tt = __builtin_amdgcn_readlane(last, 63);
             Ne = active_waves(p, Tt);
         } else {
-            ctx = last = 0;
             Tt = p.plan[p.B];
             Ne = p.plan[p.B + 1];
         }
     }
     // plan[b + 1], plan[b] and the context length of sequence b (wave-uniform)
-    __device__ __forceinline__ int end(int b) const { return regs ? __builtin_amdgcn_readlane(last, b) : p.plan[b + 1]; }
+    __device__ __forceinline__ int end(int b) const {
+        if constexpr (REGS) return __builtin_amdgcn_readlane(last, b);
+        else return p.plan[b + 1];
+    }
     __device__ __forceinline__ int begin(int b) const {
-        return regs ? (b == 0 ? 0 : __builtin_amdgcn_readlane(last, b - 1)) : p.plan[b];
+        if constexpr (REGS) return b == 0 ? 0 : __builtin_amdgcn_readlane(last, b - 1);
+        else return p.plan[b];
     }
     __device__ __forceinline__ int context(int b) const {
-        return regs ? __builtin_amdgcn_readlane(ctx, b) : ctx_of(p, b);
+        if constexpr (REGS) return __builtin_amdgcn_readlane(ctx, b);
+        else return ctx_of(p, b);
     }
     // The sequence that tile x < Tt belongs to.
     __device__ __forceinline__ int sequence_of(int x) const {
         const int lane = threadIdx.x & 63;
-        if (regs) return __builtin_ctzll(__ballot(lane < p.B && last > x));
-        int b = 0;
-        for (int b0 = 0; b0 < p.B; b0 += 64) {
-            const int bi = b0 + lane;
-            const unsigned long long m = __ballot(bi < p.B && p.plan[bi] <= x);
-            if (m == 0) break;
-            b = b0 + 63 - __builtin_clzll(m);
+        if constexpr (REGS) {
+            return __builtin_ctzll(__ballot(lane < p.B && last > x));
+        } else {
+            int b = 0;
+            for (int b0 = 0; b0 < p.B; b0 += 64) {
+                const int bi = b0 + lane;
+                const unsigned long long m = __ballot(bi < p.B && p.plan[bi] <= x);
+                if (m == 0) break;
+                b = b0 + 63 - __builtin_clzll(m);
+            }
+            return b;
         }
-        return b;
     }
 };
 
@@ -234,7 +242,7 @@ __device__ __forceinline__ void to_mt8(const u32x4* w, u32x4& h, u32x4& l) {
 // wave v owns columns [v DF / WPB, (v + 1) DF / WPB) of K, V, Q and O, the
 // partial S^T tiles meet in LDS (two barriers per tile), and every wave forms
 // the same weights.
-template <typename QE, typename CE, int DF, bool UNIFORM, int WPB = 1>
+template <typename QE, typename CE, int DF, bool UNIFORM, int WPB, bool REGS>
 __global__ __launch_bounds__(64 * WPB) void paged_partial_kernel(PagedParams p) {
     constexpr int D = DF / WPB;  // columns of this wave
     using Ty = PagedTypes<QE, CE>;
@@ -272,7 +280,7 @@ __global__ __launch_bounds__(64 * WPB) void paged_partial_kernel(PagedParams p) 
     const int hi = lane >> 5;
     const int l32 = lane & 31;
     const int w = blockIdx.x;
-    const WavePlan plan(p);
+    const WavePlan<REGS> plan(p);
     const int Tt = plan.Tt, Ne = plan.Ne;
     if (w >= Ne) return;  // no work for this wave (tiny problems)
     const int x_end = static_cast<int>(static_cast<int64_t>(w + 1) * Tt / Ne);
@@ -518,19 +526,39 @@ __global__ __launch_bounds__(64 * WPB) void paged_partial_kernel(PagedParams p) 
     }
 }
 
+// Slots i0 + i .. i0 + i + RUN - 1 (those below i0 + m) of a segment, D floats
+// apart, all read before the first is added; sl: lane l holds the sum of slot
+// i0 + l.
+template <int RUN>
+__device__ __forceinline__ void merge_run(const float* wo, int D, float sl, int i0, int i, int m, float& o, float& s) {
+    float po[RUN];
+#pragma unroll
+    for (int j = 0; j < RUN; ++j) po[j] = wo[static_cast<int64_t>(i0 + min(i + j, m - 1)) * D];
+    // (selected, not branched over: the compiler sinks loads into branches)
+#pragma unroll
+    for (int j = 0; j < RUN; ++j) {
+        const float on = o + po[j];
+        const float sn = s + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sl), min(i + j, 63)));
+        o = i + j < m ? on : o;
+        s = i + j < m ? sn : s;
+    }
+}
+
 // Sum the piece partials of one (b, query head) in slot order, then divide
-// (an empty context gives 0 / eps = 0).  Bound by memory latency: up to
-// kMergeRun slots are read before the first is added (one at a time, 8
-// sequences of 64 to 2048 tokens took 9.6 us here).
-constexpr int kMergeRun = 16;
-template <int D>
+// (an empty context gives 0 / eps = 0).  Bound by memory latency, so slots are
+// read in runs (one at a time, 8 sequences of 64 to 2048 tokens took 9.6 us
+// here), of about as many as there are: large batches have one to three a
+// segment, where runs of 16 took 9.4 us for 200 sequences of 128 to 512 tokens
+// and single slots 7.0.  With the plan's builds, whole calls: those 66.8 -> 64.9
+// us, 300 of 500 to 2000 tokens 277 -> 273, one of 16384 16.9 -> 16.1.
+template <int D, bool REGS>
 __global__ __launch_bounds__(D < 64 ? 64 : D) void paged_merge_kernel(PagedParams p) {
     const int bh = blockIdx.x;
     const int b = bh / p.Hq;
     const int hq = bh - b * p.Hq;
     const int hk = hq / p.G;
     const int d = threadIdx.x;
-    const WavePlan plan(p);
+    const WavePlan<REGS> plan(p);
     const int seg0 = plan.begin(b);
     const int n_b = (plan.end(b) - seg0) / p.Hkv;
     float o = 0.f, s = 0.f;
@@ -545,16 +573,14 @@ __global__ __launch_bounds__(D < 64 ? 64 : D) void paged_merge_kernel(PagedParam
         for (int i0 = 0; i0 < n; i0 += 64) {
             const int m = min(n - i0, 64);
             const float sl = ws[i0 + min(d & 63, m - 1)];  // lane l: the sum of slot i0 + l
-            for (int i = 0; i < m; i += kMergeRun) {
-                float po[kMergeRun];
-#pragma unroll
-                for (int j = 0; j < kMergeRun; ++j) po[j] = wo[static_cast<int64_t>(i0 + min(i + j, m - 1)) * p.D];
-#pragma unroll
-                for (int j = 0; j < kMergeRun; ++j) {
-                    if (i + j < m) {
-                        o += po[j];
-                        s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sl), i + j));
-                    }
+            if constexpr (REGS) {
+                for (int i = 0; i < m; i += 16) merge_run<16>(wo, p.D, sl, i0, i, m, o, s);
+            } else {
+                for (int i = 0; i < m;) {
+                    const int left = m - i;  // wave-uniform
+                    if (left > 8) merge_run<16>(wo, p.D, sl, i0, i, m, o, s), i += 16;
+                    else if (left > 2) merge_run<8>(wo, p.D, sl, i0, i, m, o, s), i += 8;
+                    else merge_run<2>(wo, p.D, sl, i0, i, m, o, s), i += 2;
                 }
             }
         }
@@ -562,9 +588,9 @@ __global__ __launch_bounds__(D < 64 ? 64 : D) void paged_merge_kernel(PagedParam
     if (d < p.D) p.out[b * p.os[0] + hq * p.os[1] + d * p.os[2]] = static_cast<bf16>(o / (s + kEps));
 }
 
-// Blocks of paged_partial_kernel<QE, CE, D, U, WPB> resident on the device at
+// Blocks of paged_partial_kernel<QE, CE, D, U, WPB, REGS> resident on the device at
 // once (the persistent grid), per device.
-template <typename QE, typename CE, int D, bool U, int WPB>
+template <typename QE, typename CE, int D, bool U, int WPB, bool REGS>
 int resident_waves() {
     static int cache[16] = {0};
     int dev = 0;
@@ -574,7 +600,7 @@ int resident_waves() {
         int cus = 0, per_cu = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_partial_kernel<QE, CE, D, U, WPB>, 64 * WPB,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, paged_partial_kernel<QE, CE, D, U, WPB, REGS>, 64 * WPB,
                                                          0) !=
                 hipSuccess ||
             per_cu <= 0)
@@ -584,7 +610,7 @@ int resident_waves() {
     return cache[slot];
 }
 
-template <typename QE, typename CE, int D>
+template <typename QE, typename CE, int D, bool REGS>
 int launch_paged(PagedParams prm, hipStream_t st) {
     // waves per block, each owning D / WPB columns: rows above 512 bytes are
     // split into 512-byte parts (their tile registers would not fit one wave)
@@ -594,19 +620,24 @@ int launch_paged(PagedParams prm, hipStream_t st) {
     constexpr int WPB = D / WPB_B > 256 ? D / 256 : WPB_B;
     const bool uniform = prm.P * (D / WPB * static_cast<int>(sizeof(CE)) / 16) >= 64;
     const int resident =
-        uniform ? resident_waves<QE, CE, D, true, WPB>() : resident_waves<QE, CE, D, false, WPB>();
+        uniform ? resident_waves<QE, CE, D, true, WPB, REGS>() : resident_waves<QE, CE, D, false, WPB, REGS>();
     // The plan gives work to at most Tt / per waves, and Tt is at most
     // B * Hkv * ceil(max_pages * P / kTile): no more waves are launched.
     const int64_t max_tiles = static_cast<int64_t>(prm.B) * prm.Hkv *
                               ((static_cast<int64_t>(prm.max_pages) * prm.P + kTile - 1) / kTile);
     prm.n_waves = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(resident, max_tiles / prm.per)));
-    if (prm.B > kRegSeqs) paged_plan_kernel<<<1, 256, 0, st>>>(prm);
+    if constexpr (!REGS) paged_plan_kernel<<<1, 256, 0, st>>>(prm);
     if (uniform)
-        paged_partial_kernel<QE, CE, D, true, WPB><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
+        paged_partial_kernel<QE, CE, D, true, WPB, REGS><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
     else
-        paged_partial_kernel<QE, CE, D, false, WPB><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
-    paged_merge_kernel<D><<<static_cast<unsigned>(prm.B) * prm.Hq, (prm.D + 63) / 64 * 64, 0, st>>>(prm);
+        paged_partial_kernel<QE, CE, D, false, WPB, REGS><<<prm.n_waves, 64 * WPB, 0, st>>>(prm);
+    paged_merge_kernel<D, REGS><<<static_cast<unsigned>(prm.B) * prm.Hq, (prm.D + 63) / 64 * 64, 0, st>>>(prm);
     return status_from_launch();
+}
+
+template <typename QE, typename CE, int D>
+int launch_paged(const PagedParams& prm, hipStream_t st) {
+    return prm.B <= kRegSeqs ? launch_paged<QE, CE, D, true>(prm, st) : launch_paged<QE, CE, D, false>(prm, st);
 }
 
 template <typename QE, typename CE>

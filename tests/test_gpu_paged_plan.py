@@ -57,3 +57,10 @@ def test_empty_contexts(B):
 def test_many_partials_per_segment(ctx):
     check([ctx], 2, 1, 128, ctx)
     check([ctx, 3, ctx - 40], 8, 2, 64, ctx)
+
+
+@pytest.mark.parametrize("ctx", [32, 64, 96, 8 * 32, 9 * 32 + 1, 16 * 32, 17 * 32, 25 * 32, 70 * 32])
+def test_many_partials_in_a_large_batch(ctx):
+    # past 64 sequences the merge reads a segment's partials 2, 8 or 16 at a
+    # time: one long segment of 1 to 70 partials among short ones
+    check([5] * 40 + [ctx] + [0, 33] * 13, 4, 2, 64, ctx)
