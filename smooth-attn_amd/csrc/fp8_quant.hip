@@ -8,10 +8,9 @@
 // two launches where a call per tensor takes nine (three each, the first to
 // clear the one word that its blocks meet in).
 // HBM binds the large sizes and the launches the small ones: q, k and v of a
-// [2,32/8,8192,128] forward 107 -> 86 us (31.5 us at 6.4 TB/s, then 54 us at
-// 5.6 TB/s), its whole call 945 -> 922 us; a [1,32/8,2048,128] call
-// 83 -> 63 us, then 55 (load_words_cached).  Walking the second pass backwards, towards what the first
-// read last, changed nothing.  Both passes
+// [2,32/8,8192,128] forward 103 -> 79 us, its whole call 945 -> 919 us; a
+// [1,32/8,2048,128] call 83 -> 55 us.  Walking the second pass backwards,
+// towards what the first read last, changed nothing.  Both passes
 // read 16 bytes per lane and load when x is 16-byte aligned (the remainder,
 // and unaligned inputs, element by element), several loads in flight per lane.
 #include "common.hpp"
@@ -21,15 +20,27 @@ namespace {
 
 constexpr int kQThreads = 256;
 constexpr int kMaxTensors = 4;
-// Maxima kept per tensor, so also the most blocks of the amax pass on one:
-// four per CU over all tensors.  A caller that brings one word instead of
-// kSlots has the blocks meet in it by atomicMax (non-negative floats order
-// like their bit patterns); those serialise, so that route keeps to one block
-// per CU (67M bf16: 4096 blocks 95 us, 512 blocks 64 us, 256 blocks x 8 loads
-// 62 us for both passes).
+// Maxima kept per tensor, so also the most blocks of the amax pass on one.
 constexpr unsigned kSlots = SA_FP8_AMAX_WORDS;
+// Blocks of the amax pass over all tensors.  More cost (a single tensor of
+// 2^24 fp32, 256 / 384 / 512 / 1024 blocks: 26.6 / 27.2 / 27.7 / 29.2 us; of 2^26
+// bf16 52.3 / 52.5 / 53.6 / 56.1), fewer leave q, k and v of short calls waiting
+// ([1,32/8,2048,128] 14.2 / 12.3 / 15.5 / 14.4).  A caller that brings one word
+// instead of kSlots has the blocks meet in it by atomicMax (non-negative floats
+// order like their bit patterns); those serialise, so that route keeps to one
+// block per CU.
+constexpr unsigned kAmaxBlocks = 384;
 constexpr unsigned kAmaxAtomicBlocks = 256;
+// Inputs up to this size are read through the caches, so that the second pass
+// finds there what the first has just read (nontemporal loads -> these, whole
+// calls, bf16 inputs: [1,32/8,2048,128] 61.1 -> 55.3 us, [8,32/8,1024,128] 124.7
+// -> 120.5, [1,32/8,8192,128] 467.9 -> 463.7).  Past the size of the 256 MB
+// last-level cache it finds nothing and the lines it left cost: nontemporal
+// loads and one block per CU, as -> through the caches, 268 MB 113 -> 112 us,
+// 402 MB 149 -> 165, 537 MB 196 -> 230.
+constexpr int64_t kCachedBytes = int64_t(320) << 20;
 constexpr int kAmaxUnroll = 8;
+static_assert(kAmaxBlocks <= kSlots && kAmaxAtomicBlocks <= kSlots, "one word per block");
 constexpr unsigned kQuantBlocks = 4096;
 
 struct QuantTensor {
@@ -51,19 +62,19 @@ struct QuantArgs {
 
 __global__ void fill_zero_u32(uint32_t* p) { p[0] = 0u; }
 
-// 16-byte loads that leave their lines in the caches: the second pass reads
-// what the first one has just read, from the caches for calls up to their
-// size.  Nontemporal loads -> these, whole calls (bf16 inputs):
-// [1,32/8,2048,128] 61.1 -> 55.3 us, [8,32/8,1024,128] 124.7 -> 120.5,
-// [4,16/2,3001,64] 115.4 -> 110.8, [1,32/8,8192,128] 467.9 -> 463.7,
-// [2,32/8,8192,128] (201 MB of inputs) unchanged.
-template <typename T>
-__device__ __forceinline__ void load_words_cached(const T* p, uint32_t* words) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-    words[0] = v.x;
-    words[1] = v.y;
-    words[2] = v.z;
-    words[3] = v.w;
+// 16-byte loads: nontemporal (STREAM), or leaving their lines in the caches
+// (see kCachedBytes).
+template <bool STREAM, typename T>
+__device__ __forceinline__ void load_x(const T* p, uint32_t* words) {
+    if constexpr (STREAM) {
+        load_words(p, words);
+    } else {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+        words[0] = v.x;
+        words[1] = v.y;
+        words[2] = v.z;
+        words[3] = v.w;
+    }
 }
 
 template <typename T>
@@ -87,7 +98,7 @@ __device__ __forceinline__ float block_max(float v) {
     return b;
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
     int ti = 0;
     while (ti + 1 < a.count && blockIdx.x >= a.t[ti + 1].amax_begin) ++ti;
@@ -107,7 +118,7 @@ __global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
     for (; i + (U - 1) * stride < nv; i += U * stride) {
         uint32_t w[U][4];
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_words_cached(x + (i + u * stride) * NV, w[u]);
+        for (int u = 0; u < U; ++u) load_x<STREAM>(x + (i + u * stride) * NV, w[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -115,7 +126,7 @@ __global__ __launch_bounds__(kQThreads) void amax_kernel(const QuantArgs a) {
     }
     for (; i < nv; i += stride) {
         uint32_t w[4];
-        load_words_cached(x + i * NV, w);
+        load_x<STREAM>(x + i * NV, w);
 #pragma unroll
         for (int e = 0; e < NV; ++e) m = fmaxf(m, fabsf(elem<T>(w, e)));
     }
@@ -162,7 +173,7 @@ __device__ __forceinline__ uint32_t pack_e4m3(float v0, float v1, float v2, floa
     return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(v2, v3, lo, true));
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(kQThreads) void quant_kernel(const QuantArgs a) {
     constexpr int NV = 16 / sizeof(T);  // elements per 16-byte load
     int ti = 0;
@@ -197,14 +208,14 @@ __global__ __launch_bounds__(kQThreads) void quant_kernel(const QuantArgs a) {
         int64_t i = tid0;
         for (; i + stride < nv; i += 2 * stride) {  // two loads in flight per lane
             uint32_t w0[4], w1[4];
-            load_words_cached(x + i * NV, w0);
-            load_words_cached(x + (i + stride) * NV, w1);
+            load_x<STREAM>(x + i * NV, w0);
+            load_x<STREAM>(x + (i + stride) * NV, w1);
             emit(i, w0);
             emit(i + stride, w1);
         }
         for (; i < nv; i += stride) {
             uint32_t w[4];
-            load_words_cached(x + i * NV, w);
+            load_x<STREAM>(x + i * NV, w);
             emit(i, w);
         }
         if (block == 0) {
@@ -241,7 +252,8 @@ int launch_quant(QuantArgs& a, hipStream_t st) {
     constexpr int64_t kPerBlock = kQThreads * 4 * NV;
     double total = 0;
     for (int i = 0; i < a.count; ++i) total += static_cast<double>(a.t[i].n);
-    const unsigned amax_limit = a.shared_word ? kAmaxAtomicBlocks : kSlots;
+    const bool stream = total * sizeof(T) > static_cast<double>(kCachedBytes);
+    const unsigned amax_limit = a.shared_word || stream ? kAmaxAtomicBlocks : kAmaxBlocks;
     unsigned amax_grid = 0, quant_grid = 0;
     for (int i = 0; i < a.count; ++i) {
         QuantTensor& t = a.t[i];
@@ -260,8 +272,13 @@ int launch_quant(QuantArgs& a, hipStream_t st) {
         amax_grid += t.amax_blocks = blocks(amax_limit);
         quant_grid += t.quant_blocks = blocks(kQuantBlocks);
     }
-    amax_kernel<T><<<amax_grid, kQThreads, 0, st>>>(a);
-    quant_kernel<T><<<quant_grid, kQThreads, 0, st>>>(a);
+    if (stream) {
+        amax_kernel<T, true><<<amax_grid, kQThreads, 0, st>>>(a);
+        quant_kernel<T, true><<<quant_grid, kQThreads, 0, st>>>(a);
+    } else {
+        amax_kernel<T, false><<<amax_grid, kQThreads, 0, st>>>(a);
+        quant_kernel<T, false><<<quant_grid, kQThreads, 0, st>>>(a);
+    }
     return status_from_launch();
 }
 

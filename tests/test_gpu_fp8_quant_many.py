@@ -93,3 +93,17 @@ def test_one_word_workspace_matches_many(dtype, n, offset):
         assert torch.equal(scale, want.reshape(1))
         assert torch.equal(x8[:n], want8.view(torch.uint8).reshape(-1))
         assert n > 0 or int(x8[0]) == 0x55  # nothing written
+
+
+@pytest.mark.parametrize("sizes", [((81 << 20) + 5,), (84 << 20, 1000, 7)])
+def test_inputs_past_the_caches(sizes):
+    # over 320 MiB of fp32 the passes stream: codes and scales of each tensor
+    # as alone, where it is short, and as one division per element says
+    g = torch.Generator(device=DEV).manual_seed(1)
+    xs = [torch.randn(n, generator=g, device=DEV) * 2 for n in sizes]
+    for (x8, scale), x in zip(kernels._quantize_many_to_fp8_device(*xs), xs):
+        assert float(scale) == float(x.abs().max().cpu() / 448.0)  # one fp32 division, on the CPU
+        for part in (x[:4096], x[-4096:], x[x.numel() // 2:][:4096]):
+            i = (part.data_ptr() - x.data_ptr()) // 4
+            want = (part.cpu() / scale.cpu()).clamp(-448, 448).to(torch.float8_e4m3fn)
+            assert torch.equal(x8[i:i + part.numel()].cpu().view(torch.uint8), want.view(torch.uint8))
