@@ -541,12 +541,14 @@ int chunks_for(int n_cols, int vec) {
 // 29.4 us; one [4095,4095] 43.2 / 47.8 -> 13.2 / 16.4 us; row-wise fp32 at
 // 1023 columns 91.6 -> 47.9 us, at 129 12.9 -> 9.9 us.  Below, a row fills a
 // fraction of one wave's lanes and the element kernels win: bf16 at 129
-// columns 10.4 / 12.1 vs 11.7 / 16.3 us.
-constexpr int kAnyRowBytes = 512;
-bool any_rows_ok(int64_t n_rows, int n_cols, int nch, int elem_bytes) {
+// columns 10.4 / 12.1 vs 11.7 / 16.3 us.  The causal backward of 16-bit rows
+// crosses later, at 640 bytes: element / ANY, 508 matrices of 257 rows 51.6 /
+// 53.7 us, 370 of 301 45.8 / 47.5, 128 of 511 41.3 / 32.3.
+constexpr int kAnyRowBytes = 512, kAnyCausalBwdRowBytes16 = 640;
+bool any_rows_ok(int64_t n_rows, int n_cols, int nch, int elem_bytes, int least = kAnyRowBytes) {
     const int R = split_for(nch);
     const dim3 sg = R == 8 ? split_grid<8>(n_rows) : R == 4 ? split_grid<4>(n_rows) : split_grid<1>(n_rows);
-    return n_cols * elem_bytes >= kAnyRowBytes && grid_fits(sg, dim3(64 * std::max(R, kWavesPerBlock)));
+    return n_cols * elem_bytes >= least && grid_fits(sg, dim3(64 * std::max(R, kWavesPerBlock)));
 }
 
 float eps_for_power(int power) { return kEps * static_cast<float>(1 << power); }
@@ -644,7 +646,8 @@ int launch_bwd_t(const void* x, const void* dy, void* dx, int64_t n_rows, int n_
     const bool vec_ok = (n_cols % VEC == 0) && (xs % VEC == 0) && (gs % GVEC == 0) && (dxs % VEC == 0) &&
                         aligned16(x) && aligned16(dy) && aligned16(dx);
     const int nch = chunks_for(n_cols, VEC);
-    if (!vec_ok && !any_rows_ok(n_rows, n_cols, nch, sizeof(T))) {
+    const int any_bytes = causal && sizeof(T) == 2 ? kAnyCausalBwdRowBytes16 : kAnyRowBytes;
+    if (!vec_ok && !any_rows_ok(n_rows, n_cols, nch, sizeof(T), any_bytes)) {
         if (!grid_fits(grid, block)) return SA_ERR_BAD_SHAPE;
         norm_bwd_scalar<T, TG, POWER><<<grid, block, 0, st>>>(xp, gp, dp, n_rows, n_cols, xs, gs, dxs, causal,
                                                               alpha, nat, eps);

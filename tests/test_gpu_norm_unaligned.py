@@ -44,7 +44,7 @@ def _cond(a, power):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("L,extra,offset", [(255, 0, 0), (256, 1, 0), (257, 0, 0), (505, 0, 1), (511, 0, 0), (513, 0, 0),
+@pytest.mark.parametrize("L,extra,offset", [(255, 0, 0), (256, 1, 0), (257, 0, 0), (319, 0, 0), (321, 0, 0), (505, 0, 1), (511, 0, 0), (513, 0, 0),
                                             (520, 1, 0), (1023, 0, 0), (1025, 3, 1), (2049, 0, 0), (4095, 0, 0),
                                             (4097, 0, 1), (8191, 0, 0), (8192, 1, 1)])
 @pytest.mark.parametrize("causal", [True, False])
