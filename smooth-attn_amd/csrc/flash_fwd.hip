@@ -133,12 +133,12 @@ double forward_estimate(const FlashParams& p, const SplitCosts& c, double ragged
 // that leave CUs idle or waiting for the longest block, but costs a merge and
 // more barriers per MFMA, so full grids keep KS = 1 at D = 128; at D = 64 two
 // KS = 2 blocks fit a CU (under 128 registers) and it wins over most sizes.
-// The constants (us) are fitted to measured shapes of D = 64 to 128 (bf16, T =
-// 256 .. 8192, up to 1100 blocks of 256 rows, GQA 1 to 8, windows of none to
-// most).  On the 811 of profiles/attention_fwd_key_split_us.csv the choice
-// averages 1.1% over the fastest KS at D = 72 to 128, 0.5% at D = 40 to 64 and
-// 6% at D = 32, which shares their constants; against KS = 1 throughout it takes
-// 0.84, 0.80 and 0.79 of the time, at worst 1.18.  KS = 1 / 2 / 4 in us,
+// The constants (for D <= 128, 64 and 32, about us) are fitted to the 811
+// measured shapes of profiles/attention_fwd_key_split_us.csv (bf16, T = 256 ..
+// 8192, up to 1100 blocks of 256 rows, GQA 1 to 8, windows of none to most), on
+// which the choice averages 0.5%, 0.5% and 1.0% over the fastest KS and takes
+// 0.84, 0.80 and 0.76 of the time of KS = 1 throughout, at worst 1.09, 1.17 and
+// 1.09.  KS = 1 / 2 / 4 in us,
 // D = 128: [1,32/8,512] 18.7 / 15.3 / 13.1, [1,32/8,1024] 31.4 / 23.4 / 26.2,
 // [1,32/8,2048] 58.0 / 52.4 / 69.9, [1,8,2048] 54.3 / 35.5 / 25.6,
 // [2,32/8,1024] 34.0 / 35.3 / 49.4; D = 64: [1,32/8,5760] 207 / 179 / 251.
@@ -146,13 +146,14 @@ double forward_estimate(const FlashParams& p, const SplitCosts& c, double ragged
 // their noise or lose ([1,32,8128] at D = 64, 1024 blocks, 350 / 374) and skip
 // the estimate.  KS = 4 walks tiles of 128 rows, whose 32-bit offsets bound
 // the row stride.
-constexpr ForwardCosts kForwardCosts128 = {{3.4, 2.35, 3.9, 2.99}, {6.3, 0.84, 7.5, 1.31}, {6.8, 1.16, 7.4, 1.20}, 0.03, 0.78};
+constexpr ForwardCosts kForwardCosts128 = {{6.5, 1.35, 7.7, 1.54}, {6.8, 0.78, 11.6, 1.01}, {4.7, 1.10, 9.2, 1.16}, 0.093, 1.16};
 constexpr ForwardCosts kForwardCosts64 = {{9.7, 1.99, 4.6, 3.53}, {8.3, 0.85, 3.3, 1.25}, {7.1, 1.35, 8.1, 1.15}, 0.35, 1.02};
+constexpr ForwardCosts kForwardCosts32 = {{4.0, 0.87, 0.0, 1.15}, {4.3, 0.53, 2.6, 0.53}, {4.1, 0.66, 3.1, 0.43}, 0.49, 1.0};
 int key_split_for(const FlashParams& p, int qk_bytes, int v_bytes) {
     const int64_t limit = p.dr > 32 && p.dr <= 64 ? 768 : 512;
     if (static_cast<int64_t>(p.nqb) * p.B * p.Hq > limit) return 1;
     constexpr int64_t kMaxStride4 = int64_t(1) << 23;
-    const ForwardCosts& c = p.dr > 64 ? kForwardCosts128 : kForwardCosts64;
+    const ForwardCosts& c = p.dr > 64 ? kForwardCosts128 : p.dr > 32 ? kForwardCosts64 : kForwardCosts32;
     const double e1 = forward_estimate<1>(p, c.ks1, c.ragged);
     const double e2 = forward_estimate<2>(p, c.ks2, c.ragged);
     const double e4 = p.ks[2] * qk_bytes <= kMaxStride4 && p.vs[2] * v_bytes <= kMaxStride4

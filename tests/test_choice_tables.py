@@ -29,9 +29,8 @@ def _class(D):
     return 128 if D > 64 else 64 if D > 32 else 32
 
 
-# (D <= 32 shares the constants of D = 64)
-@pytest.mark.parametrize("cls,mean,worst", [(128, 1.012, 1.28), (64, 1.006, 1.17), (32, 1.065, 1.54)])
-def test_forward_key_split(cls, mean, worst):
+@pytest.mark.parametrize("cls,mean,worst,over_one", [(128, 1.006, 1.17, 1.1), (64, 1.006, 1.17, 1.18), (32, 1.011, 1.26, 1.1)])
+def test_forward_key_split(cls, mean, worst, over_one):
     lib, cost, one = _lib.load(), [], []
     for shape, us in _table("attention_fwd_key_split_us.csv"):
         if _class(shape[4]) != cls:
@@ -42,7 +41,7 @@ def test_forward_key_split(cls, mean, worst):
     assert len(cost) > 100
     got = _over_fastest(cost)
     assert got[0] <= mean and got[1] <= worst
-    assert sum(one) / len(one) <= 0.85 and max(one) <= 1.18  # against no split at all
+    assert sum(one) / len(one) <= 0.85 and max(one) <= over_one  # against no split at all
 
 
 @pytest.mark.parametrize("kind,cls,mean,worst", [

@@ -56,8 +56,7 @@ def check(q, k, v, window):
     (TWO, 385, 128, 0), (TWO, 449, 64, 0), (TWO, 511, 32, 0), (TWO, 512, 128, 300), (TWO, 513, 72, 0),
     (TWO, 500, 128, 450)])
 def test_key_split_matches_oracle(dtype, heads, T, D, window):
-    # (a window of 33 leaves blocks of 640 rows too little to share out four ways)
-    assert takes(heads, T, D, window, 2 if (heads, T, window) == (FOUR, 640, 33) else GROUPS[heads])
+    assert takes(heads, T, D, window, GROUPS[heads])
     check(*qkv(heads, T, D, dtype, T + D), window)
 
 
