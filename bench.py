@@ -732,12 +732,12 @@ def bench_norm_rotating(torch, sa):
 
 # ---------------------------------------------------------------------------
 # CPU baselines: the reference's eager CPU path, restated in oracle/ (fp32
-# torch), on the host cores of the GPU box.
+# torch), on the host cores of the machine.
 # ---------------------------------------------------------------------------
 def cpu_threads(torch):
     """Threads for the CPU legs: the cores this process may run on
     (sched_getaffinity), capped by OMP_NUM_THREADS when the environment sets
-    it (the GPU box grants one GPU's job 16 threads and sets it so).
+    it (machines that share cores among jobs set it to the job's share).
     Returns the thread count used and a description of the host."""
     try:
         affinity = len(os.sched_getaffinity(0))
